@@ -419,8 +419,8 @@ struct aq_state {
     uint32_t *ids = nullptr, *amax = nullptr, *drafts = nullptr, *emitted = nullptr, *info = nullptr, *prompt = nullptr,
              *shifted = nullptr;
     void *amax_scratch = nullptr;
-    float *attn_sc = nullptr; // attention score rows [T][n_head][attn_sc_stride], when contexts outgrow the LDS
-    size_t attn_sc_stride = 0;
+    float *attn_sc = nullptr; // attention score rows [attn_sc_rows][n_head][attn_sc_stride], for long contexts
+    size_t attn_sc_stride = 0, attn_sc_rows = 0;
     uint32_t *pinned = nullptr; // host, 64 words
     aq_sampler *sp = nullptr;   // the sampler of the running sampled call (null: greedy)
     float *q_dense = nullptr;   // k x vocab: each draft's dense distribution (sampled rounds)
@@ -674,11 +674,13 @@ int mixer(aq_state *s, const DevLayer &L, size_t t, size_t start_pos, KvDev *kv,
         a.rd = (int)c.rope_dim;
         a.gsc = s->attn_sc;
         a.gsc_stride = s->attn_sc_stride;
-        // the whole chunk in one launch while its scores fit the LDS; past that, pieces of at most MAX_ROWS rows
-        // (the score rows a context past the LDS keeps in device memory are that many), each piece's K/V rows
-        // appended before the next piece attends to them
+        // pieces of as many rows as there are score rows where those are in device memory (the split core, and
+        // contexts past the single-launch core's LDS), each piece's K/V rows appended before the next piece attends
+        // to them; else the whole chunk in one launch
         const size_t qw = 2 * (size_t)c.n_head * c.head_dim, kw = kv->stride, ow = (size_t)c.n_head * c.head_dim;
-        const size_t piece = kv->len + t <= attn_lds_positions((int)c.head_dim) ? t : (size_t)MAX_ROWS;
+        const bool split = s->attn_sc && kv->len + t >= (size_t)ATTN_SPLIT_MIN && c.head_dim % 64 == 0;
+        const size_t piece = split || kv->len + t > attn_lds_positions((int)c.head_dim) ? s->attn_sc_rows : t;
+        AQ_REQUIRE(piece > 0, "attention: no score rows for this context");
         for (size_t r0 = 0; r0 < t; r0 += piece) {
             const size_t tr = t - r0 < piece ? t - r0 : piece;
             AttnArgs ap = a;
@@ -1050,11 +1052,14 @@ int aq_state_new(aq_model *m, uint32_t spec_k, uint32_t max_pos, aq_state **out)
             AQ_S(dalloc_t(s, T * nv, &s->sv_b[i]));
         }
     }
-    // score rows in device memory when a context can outgrow the attention kernel's LDS (the MTP's cache is the
-    // longest: cap + T rows)
-    if (cap + 2 * T > attn_lds_positions((int)c.head_dim)) {
-        s->attn_sc_stride = cap + 2 * T;
-        AQ_S(dalloc_t(s, T * c.n_head * s->attn_sc_stride, &s->attn_sc));
+    // score rows in device memory for contexts the split core takes (head_dim of whole 64s), or that can outgrow the
+    // single-launch core's LDS (the MTP's cache is the longest: cap + T rows): a prompt chunk's rows, fewer where
+    // those pass 192 MB, a verify batch's at least
+    if ((cap + 2 * T >= (size_t)ATTN_SPLIT_MIN && c.head_dim % 64 == 0) || cap + 2 * T > attn_lds_positions((int)c.head_dim)) {
+        s->attn_sc_stride = (cap + 2 * T + 63) / 64 * 64;
+        const size_t fit = ((size_t)192 << 20) / (c.n_head * s->attn_sc_stride * sizeof(float));
+        s->attn_sc_rows = fit < T ? T : (fit > TP ? TP : fit);
+        AQ_S(dalloc_t(s, s->attn_sc_rows * c.n_head * s->attn_sc_stride, &s->attn_sc));
     }
     if (m->has_mtp) {
         s->mtp_kv.cap = cap + T;

@@ -1240,6 +1240,7 @@ int launch_attention(const AttnArgs &a, hipStream_t stream) {
     if (rc) return rc;
     AQ_REQUIRE(!a.out_q8k || (a.hd == 256 && a.q8k.qs && a.q8k.n == (size_t)a.nh * 256 && a.q8k.ncols >= (size_t)a.t),
                "attention: Q8_K output needs head_dim 256 and a buffer of t rows of nh * 256");
+    if (attn_split_fits(a)) return launch_attention_split(a, stream);
     if (a.base + a.t <= attn_lds_positions(a.hd)) {
         const size_t shmem = (a.hd + a.base + a.t + 32) * sizeof(float);
         hipLaunchKernelGGL(attn_core_kernel<false>, dim3((unsigned)a.nh, (unsigned)a.t), dim3(256), shmem, stream, a);
