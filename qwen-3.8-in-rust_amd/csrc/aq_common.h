@@ -130,6 +130,12 @@ struct Weight {
 //           d   ncols x nb f32; bs ncols x nb x 16 i16 (group sums); q8s ncols x nb x 8 i16 (sub-block sums)
 //   Q8_0  : q0  ncols x n int8 (natural order); d0 ncols x n/32 f32 (the f16 scale widened); h0 the f16 bits;
 //           s0  ncols x n/32 i32 (sum of the block's codes, for the Q4_0 -8 offset)
+//   Q8_K for the many-column products (buffers of more than 8 columns; null: not written), super-block-major, `gcap` the
+//   buffer's columns rounded up to 16, `gcol` the column of the buffer that this view's column 0 is:
+//           gh  f16 codes, each matrix-core operand of 16 columns one contiguous run (act_gh): per block, lane slot
+//               and 16 columns, [g][column][8]: the elements of sub-blocks 2g, 2g + 1, each the lane's four in the
+//               order b = 0, 2, 1, 3 (in which the weights' packed nibbles unpack)
+//           gm  per block and 16 columns (act_gm): the columns' 16 f16 group sums (|.| <= 2032: exact), then their f32 d
 struct Act {
     size_t n = 0, ncols = 0, nb = 0, nb32 = 0;
     float *f32 = nullptr;
@@ -140,9 +146,24 @@ struct Act {
     float *d0 = nullptr;
     uint16_t *h0 = nullptr;
     int32_t *s0 = nullptr;
+    uint16_t *gh = nullptr;
+    uint8_t *gm = nullptr;
+    size_t gcap = 0, gcol = 0;
     void *base = nullptr;
     int device = 0;
 };
+
+// Where column col's eight f16 codes of k-group g (sub-blocks 2g, 2g + 1) of lane slot `slot` start in Act::gh.
+__host__ __device__ inline size_t act_gh(size_t gcap, size_t blk, int slot, size_t col, int g) {
+    return (((blk * 8 + slot) * (gcap / 16) + col / 16) * 64 + (size_t)g * 16 + col % 16) * 8;
+}
+
+// Where the 16 columns' record of block blk that holds column col starts in Act::gm; column c = col % 16 of it: group
+// sums at 32 c, d at 512 + 4 c.
+constexpr int ACT_GM = 16 * 32 + 16 * 4;
+__host__ __device__ inline size_t act_gm(size_t gcap, size_t blk, size_t col) {
+    return (blk * (gcap / 16) + col / 16) * ACT_GM;
+}
 
 // Every device and pinned-host allocation of the library goes through these two, which count it
 // (aq_alloc_counts: what shows that a decode step or a speculative round allocates nothing).

@@ -3,25 +3,32 @@
 // column dot bit for bit: the integer lane sums are exact and each output's f32 chains advance super-block by
 // super-block (block by block for Q8_0 / Q4_0) in the reference's order.
 //
-// K-quants x Q8_K (kdot.rs:37-140, 176-333) on v_mfma_i32_16x16x32_i8. The reference's lane l of a super-block is
+// K-quants x Q8_K (kdot.rs:37-140, 176-333) on v_mfma_f32_16x16x32_f16. The reference's lane l of a super-block is
 // the 32 elements 32s + 4l + b (s = sub-block, b = 0..3), and its sum is sum_s sc[s] * sum_b q * x. One matrix-core
 // product over K = 32 covers exactly lane l: k-group g of the operands (lanes 16g .. 16g + 15) takes sub-blocks 2g and
-// 2g + 1, four elements each. Q4_K / Q5_K (v_mfma_i32_16x16x32_i8): the scale goes into the weight operand as digits
-// small enough that digit * code fits an int8 (6-bit scales in two base-8 digits, codes <= 15; three base-4 digits,
-// codes <= 31), the digit products chained through the accumulator (c = digit_hi product; c = c * base + next
-// digit's product ...). Q6_K (v_mfma_f32_16x16x32_f16): the signed 8-bit group scale sc = 16 hi + lo goes into two
-// f16 weight operands q * lo and q * hi (unsigned codes <= 63: both exact in f16), the activation codes as f16, both
-// sums exact in f32, taken to i32 as 16 * hi_sum + lo_sum, and the reference's -32 offset taken from the activation's
-// 16-element group sums into lane l exactly as kdot.rs:125-129 does (the reference's lane split of it). Either
-// way the result is the exact lane sum for a 16-row x 16-column tile. The f32 part then runs per output in the lanes
-// that hold it (4 rows x 1 column per lane): acc[l] += (dx * d) * f32(sumi[l]), accm[i] += (-dx * dmin) *
-// f32(prod[i]), no FMA, and reduce8(acc) [+ reduce4(accm)] at the end.
+// 2g + 1, four elements each. Q4_K / Q5_K: the weight operand is q * sc (codes <= 31, scales <= 63: at most 1953, exact
+// in f16), the activation codes as f16 (the quantiser writes them so: Act::gh), every partial sum an integer below
+// 2^23, exact in f32 - the product returns f32(sumi[l]), nothing to convert. Q6_K: the signed 8-bit group scale
+// sc = 16 hi + lo goes into two f16 operands q * lo and q * hi (unsigned codes <= 63: exact), the reference's -32 offset
+// enters the hi sum as -2 (bs[2l] sc[2l] + bs[2l + 1] sc[2l + 1]) (kdot.rs:125-129, the reference's lane split of it; a
+// K = 4 product of the group sums, |.| <= 2032, exact in f16), and fma(16, hi sum, lo sum) rounds the exact integer
+// once, as the reference's conversion does. The products that the f32 chains start from come from the matrix cores
+// too: d = dx * d and -dx * dmin of a 16 x 64 tile are one K = 1 f32 outer product each (rounded once, no FMA), and
+// the Q4_K / Q5_K min sums prod[i] one K = 4 product of the mins and the group sums.
 //
 // Q8_0 / Q4_0 x Q8_0 (dot.rs:29-66): one product over K = 32 is one block's exact i32 sum for the tile (Q4_0: the
 // unsigned codes, less 8 * the activation block's code sum), then acc += (dw * dx) * f32(isum) per output.
 //
-// Work: a wave owns 16 rows x 16 columns for all of K (its super-block's loads issued one step ahead); a 256-thread
-// work-group the same 16 rows x 64 columns. Rows and columns past the ends are read clamped and not written.
+// Work (K-quants): a work-group of eight waves owns two 16-row tiles x CT 16-column tiles; wave (rt, w) takes the lane
+// slots w and w + 4 (and min lane w) of row tile rt, for all of K. The eight lane chains are independent until the final
+// reduction, so nothing passes between the waves before that, and each weight code is unpacked once per work-group
+// (with a wave per column tile, as the Q8_0 / Q4_0 kernel below has it, every code is unpacked four times: Q4_K 388
+// vector instructions per 16 x 16 x 256 step, of which 112 are the f32 chains; here ~150 per 16 x 64 x 256 step and
+// wave, 96 of them the chains). Two row tiles share the activation operands, which come through the LDS by direct copies
+// several steps ahead: a wave's loads return in order, so operands loaded straight into registers wait for the weights'
+// memory latency. It is bound by the waves' instruction issue, then by the copies. Measured, 64 columns: Q4_K
+// 17408 x 5120 94 -> 56 us, Q6_K 5120 x 17408 211 -> 87, Q5_K 5120 x 6144 45 -> 26, Q4_K 10240 x 5120 -> 35; 37 columns:
+// Q6_K 5120 x 17408 208 -> 73 us.
 #include "aq_common.h"
 
 #include <atomic>
@@ -41,43 +48,13 @@ __device__ __forceinline__ float h2f(uint32_t bits16) {
     __builtin_memcpy(&f, &h, 2);
     return (float)f;
 }
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-// Bytes of x times a small factor f, per byte (every product < 256, so no carry leaves its byte): one packed 16-bit
-// multiply with f in both halves.
-__device__ __forceinline__ uint32_t mul_bytes(uint32_t x, uint32_t f) {
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, x) * __builtin_bit_cast(u16x2, f * 0x00010001u));
-}
-
-// f16 operands of the matrix-core f16 product (Q6_K). Small integers are exact in f16 (|v| <= 2048, and multiples of
-// 2^k up to 2048 * 2^k), the products of two f16 are exact in f32 and every partial sum of a lane (an integer below
-// 2^24 in magnitude) is exact in f32, so v_mfma_f32_16x16x32_f16 returns the exact integer lane sums as floats.
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint32_t h2bits(float a, float b) {
-    return __builtin_bit_cast(uint32_t, f16x2{(_Float16)a, (_Float16)b});
-}
-// Unsigned bytes 0, 1 (k = 0) or 2, 3 (k = 1) of w as the f16 pair (1024 + byte): the byte under an exponent of 2^10.
-__device__ __forceinline__ uint32_t magic_pair(uint32_t w, int k) {
-    return __builtin_amdgcn_perm(0x64646464u, w, k == 0 ? 0x04010400u : 0x04030402u);
-}
-// a * b + c on f16 pairs, one rounding (v_pk_fma_f16): exact whenever the result is representable.
-__device__ __forceinline__ uint32_t h2fma(uint32_t a, uint32_t b, uint32_t c) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b),
-                                                                  __builtin_bit_cast(f16x2, c)));
-}
-// Eight signed activation codes (bytes of x, in k order) as f16: (1024 + 128 + x) - 1152.
-__device__ __forceinline__ f16x8 codes_f16(uint64_t x) {
-    const uint32_t w0 = (uint32_t)x ^ 0x80808080u, w1 = (uint32_t)(x >> 32) ^ 0x80808080u;
-    const f16x2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-    const f16x2 p0 = __builtin_bit_cast(f16x2, magic_pair(w0, 0)) + off, p1 = __builtin_bit_cast(f16x2, magic_pair(w0, 1)) + off;
-    const f16x2 p2 = __builtin_bit_cast(f16x2, magic_pair(w1, 0)) + off, p3 = __builtin_bit_cast(f16x2, magic_pair(w1, 1)) + off;
-    return __builtin_bit_cast(f16x8, uint4{__builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1),
-                                           __builtin_bit_cast(uint32_t, p2), __builtin_bit_cast(uint32_t, p3)});
-}
-__device__ __forceinline__ f32x4 mma_f16(f16x8 a, f16x8 b) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-}
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct GemmArgs {
     const uint8_t *qa, *qb, *sc, *dm;
@@ -88,20 +65,14 @@ struct GemmArgs {
     const int16_t *xbs, *xq8s;
     const int32_t *xs0;
     size_t n;
+    // the many-column Q8_K form (Act::gh, gm; gcap columns)
+    const uint16_t *gh;
+    const uint8_t *gm;
+    uint32_t gcap;
+    int nfull; // K-quants: work-groups over all column tiles; those past them take one each
     float *y;
     const float *resid;
 };
-
-__device__ __forceinline__ int sdot2(uint32_t a, uint32_t b) {
-    typedef short s16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_amdgcn_sdot2(__builtin_bit_cast(s16x2, a), __builtin_bit_cast(s16x2, b), 0, false);
-}
-// Signed bytes k, k + 1 of w (k = 0 or 2) as an i16 pair: a byte permute of (w << 8, w) whose sign-fill selectors
-// (10 / 11: bit 15 / 31 of the first source, 8 / 9: of the second) supply each byte's sign.
-__device__ __forceinline__ uint32_t i8pair(uint32_t w, uint32_t w8, int k) {
-    return __builtin_amdgcn_perm(w8, w, k == 0 ? 0x08010A00u : 0x09030B02u);
-}
-
 
 // ---- LDS staging ----
 // Operands reach the LDS by direct global-to-LDS copies (global_load_lds_*: each active lane's 16 or 4 bytes land at
@@ -111,6 +82,7 @@ __device__ __forceinline__ uint32_t i8pair(uint32_t w, uint32_t w8, int k) {
 // landed; a work-group barrier after the wait makes every wave's copies of that step visible and, at the same
 // time, frees the buffer read one step earlier for the next copies.
 constexpr int GEMM_STAGES = 3;
+constexpr int GEMM_CUS = 256;
 
 __device__ __forceinline__ void dma16(uint32_t lds, const void *g) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(g) : "memory", "m0");
@@ -126,279 +98,357 @@ __device__ __forceinline__ void wait_vm_barrier() {
 }
 __device__ __forceinline__ uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
-// One super-block step of a K-quant work-group (16 rows, 4 waves x 16 columns) in the LDS, in 16-byte units:
-//   weight codes: unit c * 4 + k = byte chunk c of row tile k (rows r0 + 4k .. + 3) — the four tiles interleaved,
-//     qa (32 chunks a tile), then qb (Q5_K 8, Q6_K 16 chunks a tile);
-//   scale records: unit W_UNITS - 16 + i = row r0 + i's 16-byte record; Q6_K then the 4 tiles' f16 d (8 B each);
-//   per wave: codes unit q * 16 + c = byte chunk q of column c's super-block (c = 0..15); f32 dx per column;
-//     Q4_K / Q5_K the 8 sub-block sums (16 B) per column, Q6_K the 16 group sums (32 B).
+// ---- K-quants ----
+__device__ __forceinline__ f16x2 bits2(uint32_t w) { return __builtin_bit_cast(f16x2, w); }
+__device__ __forceinline__ f16x2 splat2(float v) { return f16x2{(_Float16)v, (_Float16)v}; }
+// Two unsigned bytes of w (byte selectors of v_perm_b32 in the low and high half) as the f16 pair 1024 + byte.
+template <uint32_t SEL>
+__device__ __forceinline__ f16x2 magic2(uint32_t w) {
+    return bits2(__builtin_amdgcn_perm(0x64646464u, w, SEL));
+}
+// (x & mask) | base in one instruction (one operand of the three may be scalar).
+__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t base) {
+    uint32_t r;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "s"(mask), "v"(base));
+    return r;
+}
+__device__ __forceinline__ f16x2 fma2(f16x2 a, f16x2 b, f16x2 c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ f16x8 cat(f16x2 a, f16x2 b, f16x2 c, f16x2 d) {
+    return f16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+// A wave's raw weights of one super-block: lane (li, g) holds row li's codes of lane slots w and w + 4 for sub-blocks 2g
+// and 2g + 1, and row li's scale record.
 template <int T>
-struct KqStage { // every W_UNITS / 4 <= 64: one weight copy per wave
-    static constexpr int QB_UNITS = T == AQ_TYPE_Q4_K ? 0 : (T == AQ_TYPE_Q5_K ? 32 : 64);
-    static constexpr int W_UNITS = 128 + QB_UNITS + 16;
-    static constexpr int WL = W_UNITS / 4; // weight units per wave
-    static constexpr int WB = W_UNITS * 16 + (T == AQ_TYPE_Q6_K ? 32 : 0);
-    static constexpr int XSUM = T == AQ_TYPE_Q6_K ? 512 : 256;
-    static constexpr int XB = 4096 + 64 + XSUM;
-    static constexpr int BYTES = WB + 4 * XB;
-    static constexpr int NDMA = T == AQ_TYPE_Q6_K ? 8 : 7; // copies per wave per step
+struct KqRaw {
+    uint32_t c[T == AQ_TYPE_Q4_K ? 2 : (T == AQ_TYPE_Q5_K ? 4 : 6)];
+    u32x4 rec;
+    uint32_t d6;
+};
+// Its matrix-core weight operands.
+struct KqOps {
+    f16x8 lo[2], hi[2]; // lane slots w, w + 4 (hi: Q6_K)
+    f16x4 m[2];         // the mins, or the Q6_K group scales of lanes w and w + 4
+    float d, dmin;
 };
 
-template <int T>
-__device__ __forceinline__ void kq_issue(const GemmArgs &a, uint32_t buf, size_t sb, int r0, int c0w, int wave,
-                                         int lane) {
-    using S = KqStage<T>;
-    const size_t nb = (size_t)a.nb;
-    if (lane < S::WL) {
-        const int u = wave * S::WL + lane;
-        const uint8_t *src;
-        if (u < 128) {
-            src = a.qa + kq_tile((size_t)min(r0 + 4 * (u & 3), a.rows - 1), sb, nb) * 512 + (size_t)(u >> 2) * 16;
-        } else if (u < 128 + S::QB_UNITS) {
-            const int v = u - 128;
-            src = a.qb + kq_tile((size_t)min(r0 + 4 * (v & 3), a.rows - 1), sb, nb) * (S::QB_UNITS * 4) +
-                  (size_t)(v >> 2) * 16;
-        } else {
-            src = a.sc + kq_sc_off((size_t)min(r0 + u - 128 - S::QB_UNITS, a.rows - 1), sb, nb);
-        }
-        dma16(uni(buf + (uint32_t)(wave * S::WL * 16)), src);
-    }
-    if constexpr (T == AQ_TYPE_Q6_K) {
-        if (lane < 2) {
-            const int d = 2 * wave + lane; // tile d >> 1, its rows 2 (d & 1) .. + 1
-            dma4(uni(buf + (uint32_t)(S::W_UNITS * 16 + wave * 8)),
-                 a.dm + kq_tile((size_t)min(r0 + 4 * (d >> 1), a.rows - 1), sb, nb) * 8 + 4 * (d & 1));
-        }
-    }
-    const uint32_t xw = buf + (uint32_t)(S::WB + wave * S::XB);
-    const size_t col = (size_t)min(c0w + (lane & 15), a.ncols - 1);
-    const int8_t *xs = a.xq + col * a.n + sb * 256;
-#pragma unroll
-    for (int i = 0; i < 4; i++) dma16(uni(xw + (uint32_t)(i * 1024)), xs + (size_t)(i * 4 + (lane >> 4)) * 16);
-    if (lane < 16) dma4(uni(xw + 4096), a.xd + col * nb + sb);
-    if constexpr (T == AQ_TYPE_Q6_K) {
+// One super-block step in the LDS. Per row tile its four 4-row weight tiles, each as in memory: qa (512 B), qb (Q5_K
+// 128 B, Q6_K 256 B), the four 16-byte scale records (a stride of 16 or 48 banks: the operand reads meet no bank
+// conflicts); Q6_K then the tiles' f16 d (8 B each). Activations: per lane slot and column tile the operand's 1 KB run;
+// the column tiles' group sums and d as in memory (ACT_GM B each).
+template <int T, int CT>
+struct KqStage {
+    static constexpr int QB = T == AQ_TYPE_Q4_K ? 0 : (T == AQ_TYPE_Q5_K ? 128 : 256);
+    static constexpr int TB = 512 + QB + 64, WL = TB / 16;           // a 4-row tile: bytes, lanes of its one copy
+    static constexpr int WB = 4 * TB + (T == AQ_TYPE_Q6_K ? 32 : 0); // a 16-row tile
+    static constexpr int XB = 2 * WB, GM = XB + 8 * CT * 1024, BYTES = GM + 4 * ACT_GM;
+    static constexpr int NDMA = CT + 2 + (T == AQ_TYPE_Q6_K ? 1 : 0); // copies per wave per step
+    // stages: as many as the CU's 160 KB hold for one work-group per CU at three and four column tiles, two below
+    static constexpr int LDS = CT >= 3 ? 163840 : 81920;
+    static constexpr int RING = LDS / BYTES < 6 ? LDS / BYTES : 6;
+    static_assert(RING >= 3, "stages");
+};
+
+// A wave's copies of successive steps: running source addresses (each lane's own), and the stage to fill.
+template <int T, int CT>
+struct KqCopier {
+    using S = KqStage<T, CT>;
+    const uint8_t *w, *dm, *m; // weights, Q6_K f16 d, group sums
+    const uint16_t *x;
+    uint32_t wstride, xstride, mstride; // bytes, f16, bytes per step
+    uint32_t lds0, wo, mo, xo, dofs, buf;
+    int lane;
+
+    __device__ __forceinline__ KqCopier(const GemmArgs &a, uint32_t lds, int r0, int ct0, int wave, int lane_) {
+        lane = lane_;
+        const int rt = wave >> 2, w4 = wave & 3;
+        const size_t t = kq_tile((size_t)min(r0 + 16 * rt + 4 * w4, a.rows - 1), 0, (size_t)a.nb);
+        // wave w4 copies 4-row tile w4 of its row tile
         if (lane < 32) {
-            const size_t c2 = (size_t)min(c0w + (lane >> 1), a.ncols - 1);
-            dma16(uni(xw + 4160), a.xbs + (c2 * nb + sb) * 16 + 8 * (lane & 1));
+            w = a.qa + t * 512 + lane * 16;
+            wstride = 512;
+        } else if (lane < 32 + S::QB / 16) {
+            w = a.qb + t * S::QB + (lane - 32) * 16;
+            wstride = S::QB;
+        } else {
+            w = a.sc + t * 64 + (min(lane, S::WL - 1) - 32 - S::QB / 16) * 16;
+            wstride = 64;
         }
-    } else {
-        if (lane < 16) dma16(uni(xw + 4160), a.xq8s + (col * nb + sb) * 8);
+        dm = a.dm + t * 8 + 4 * (lane & 1);
+        // lane slot `wave` of every column tile; column tile `wave`'s group sums (repeated past the last tile)
+        x = a.gh + act_gh(a.gcap, 0, wave, 16 * (size_t)ct0, 0) + 8 * lane;
+        xstride = a.gcap * 256;
+        const int ct = min(wave, CT - 1);
+        m = a.gm + act_gm(a.gcap, 0, 16 * (size_t)(ct0 + ct)) + 16 * min(lane, ACT_GM / 16 - 1);
+        mstride = a.gcap / 16 * ACT_GM;
+        lds0 = buf = lds;
+        wo = (uint32_t)(rt * S::WB + w4 * S::TB);
+        dofs = (uint32_t)(rt * S::WB + 4 * S::TB + w4 * 8);
+        xo = (uint32_t)(S::XB + wave * CT * 1024);
+        mo = (uint32_t)(S::GM + ct * ACT_GM);
+    }
+    __device__ __forceinline__ void issue() {
+        if (lane < S::WL) dma16(buf + wo, w);
+        if constexpr (T == AQ_TYPE_Q6_K) {
+            if (lane < 2) dma4(buf + dofs, dm);
+            dm += 8;
+        }
+        // the column tiles' runs are contiguous on both sides: one LDS base, the instruction's offset moves both
+        if constexpr (CT == 1)
+            dma16(buf + xo, x);
+        else if constexpr (CT == 2)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+                         "global_load_lds_dwordx4 %1, off offset:1024" ::"s"(buf + xo), "v"(x) : "memory", "m0");
+        else if constexpr (CT == 3)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+                         "global_load_lds_dwordx4 %1, off offset:1024\n\tglobal_load_lds_dwordx4 %1, off offset:2048"
+                         ::"s"(buf + xo), "v"(x) : "memory", "m0");
+        else
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
+                         "global_load_lds_dwordx4 %1, off offset:1024\n\tglobal_load_lds_dwordx4 %1, off offset:2048\n\t"
+                         "global_load_lds_dwordx4 %1, off offset:3072" ::"s"(buf + xo), "v"(x) : "memory", "m0");
+        if (lane < ACT_GM / 16) dma16(buf + mo, m);
+        w += wstride;
+        x += xstride;
+        m += mstride;
+        buf = buf + S::BYTES == lds0 + S::RING * S::BYTES ? lds0 : buf + S::BYTES;
+    }
+};
+
+// CT: 16-column tiles of the work-group (1..4).
+template <int T, int CT>
+__device__ __forceinline__ void kq_gemm_body(const GemmArgs &a, uint8_t *gm_lds, const int r0, const int ct0) {
+    using S = KqStage<T, CT>;
+    constexpr bool Q6 = T == AQ_TYPE_Q6_K;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int rt = wave >> 2, w = wave & 3;
+    const int g = lane >> 4, li = lane & 15, k4 = li >> 2, r4 = li & 3;
+    const int nb = a.nb, c0 = 16 * ct0;
+    const uint32_t magic = 0x64006400u; // 2^10's exponent in both halves: or-ed with packed integers, 1024 + v
+
+    auto unpack = [&](KqOps &p, const KqRaw<T> &k) {
+        if constexpr (Q6) {
+            // group scales of sub-blocks 2g, 2g + 1: byte 0 = 2g lanes 0-3, 1 = 2g lanes 4-7, 2 and 3 the same of 2g + 1
+            const uint32_t sw = g == 0 ? k.rec[0] : g == 1 ? k.rec[1] : g == 2 ? k.rec[2] : k.rec[3];
+            const uint32_t l4 = sw & 0x0F0F0F0Fu, h4 = ((sw ^ 0x80808080u) >> 4) & 0x0F0F0F0Fu;
+            // pairs (lanes 0-3, lanes 4-7) of sub-blocks 2g and 2g + 1
+            const f16x2 la = magic2<0x04010400u>(l4) + splat2(-1024.0f), lb = magic2<0x04030402u>(l4) + splat2(-1024.0f);
+            const f16x2 ha = magic2<0x04010400u>(h4) + splat2(-1032.0f), hb4 = magic2<0x04030402u>(h4) + splat2(-1032.0f);
+            const f16x2 cla = la * splat2(-1024.0f), clb = lb * splat2(-1024.0f);
+            const f16x2 cha = ha * splat2(-1024.0f), chb = hb4 * splat2(-1024.0f);
+            const int sh = 4 * (g & 1);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint32_t wa = k.c[2 * h] >> sh, wb = k.c[2 * h + 1] >> sh, wh = k.c[4 + h] >> sh;
+                const uint32_t wa8 = wa >> 8, wb8 = wb >> 8, wh8 = wh >> 8;
+                const f16x2 p0 = bits2(and_or(wa, 0x000F000Fu, magic) | ((wh & 0x00030003u) << 4));
+                const f16x2 p1 = bits2(and_or(wa8, 0x000F000Fu, magic) | ((wh8 & 0x00030003u) << 4));
+                const f16x2 p2 = bits2(and_or(wb, 0x000F000Fu, magic) | ((wh & 0x000C000Cu) << 2));
+                const f16x2 p3 = bits2(and_or(wb8, 0x000F000Fu, magic) | ((wh8 & 0x000C000Cu) << 2));
+                const f16x2 fl = f16x2{la[h], la[h]}, gl = f16x2{cla[h], cla[h]}, fl2 = f16x2{lb[h], lb[h]}, gl2 = f16x2{clb[h], clb[h]};
+                const f16x2 fh = f16x2{ha[h], ha[h]}, gh = f16x2{cha[h], cha[h]}, fh2 = f16x2{hb4[h], hb4[h]}, gh2 = f16x2{chb[h], chb[h]};
+                p.lo[h] = cat(fma2(p0, fl, gl), fma2(p1, fl, gl), fma2(p2, fl2, gl2), fma2(p3, fl2, gl2));
+                p.hi[h] = cat(fma2(p0, fh, gh), fma2(p1, fh, gh), fma2(p2, fh2, gh2), fma2(p3, fh2, gh2));
+            }
+            // -2 sc of groups 2w, 2w + 1 (lane w) and 2w + 8, 2w + 9 (lane w + 4): w uniform
+            const uint32_t ow = (w & 1) ? 0x00030002u : 0x00010000u; // bytes of the word
+            const uint32_t swo0 = w < 2 ? k.rec[0] : k.rec[1], swo1 = w < 2 ? k.rec[2] : k.rec[3];
+            auto m2 = [&](uint32_t word) { // -2 * the two signed bytes, as f16
+                const uint32_t u = word ^ 0x80808080u;
+                const f16x2 v = bits2(__builtin_amdgcn_perm(0x64646464u, u, 0x04000400u + ow)) + splat2(-1152.0f);
+                return v * splat2(-2.0f);
+            };
+            const f16x2 o0 = m2(swo0), o1 = m2(swo1);
+            const _Float16 z = (_Float16)0.0f;
+            p.m[0] = f16x4{o0[0], o0[1], z, z};
+            p.m[1] = f16x4{z, z, o1[0], o1[1]};
+            p.d = h2f(k.d6);
+        } else {
+            const uint32_t x = k.rec[0], y = k.rec[1], z = k.rec[2], u = k.rec[3];
+            // 6-bit scales of sub-blocks 2g, 2g + 1 (quant.rs:45-51): bytes 2g, 2g + 1 of the low or high word
+            const uint32_t sc_lo = y & 0x3F3F3F3Fu, sc_hi = (u & 0x0F0F0F0Fu) | ((y >> 2) & 0x30303030u);
+            const uint32_t scw = (g < 2 ? sc_lo : sc_hi) >> (16 * (g & 1));
+            // (s0, s1 / 16) and -1024 times it: (1024 + q) s0 - 1024 s0 and (1024 + 16 q) s1 / 16 - 64 s1, both exact
+            const f16x2 s = (magic2<0x04010400u>(scw) + splat2(-1024.0f)) * f16x2{(_Float16)1.0f, (_Float16)0.0625f};
+            const f16x2 cs = s * splat2(-1024.0f);
+            const f16x2 s0 = f16x2{s[0], s[0]}, s1 = f16x2{s[1], s[1]}, q0 = f16x2{cs[0], cs[0]}, q1 = f16x2{cs[1], cs[1]};
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const uint32_t v = k.c[h], v8 = v >> 8;
+                if constexpr (T == AQ_TYPE_Q4_K) {
+                    p.lo[h] = cat(fma2(bits2(and_or(v, 0x000F000Fu, magic)), s0, q0),
+                                  fma2(bits2(and_or(v8, 0x000F000Fu, magic)), s0, q0),
+                                  fma2(bits2(and_or(v, 0x00F000F0u, magic)), s1, q1),
+                                  fma2(bits2(and_or(v8, 0x00F000F0u, magic)), s1, q1));
+                } else {
+                    const uint32_t t = k.c[2 + h] >> (2 * g), t8 = t >> 8; // bits 0, 1 of each byte: sub-blocks 2g, 2g + 1
+                    const f16x2 b0 = bits2(and_or(v, 0x000F000Fu, magic) | ((t & 0x00010001u) << 4));
+                    const f16x2 b1 = bits2(and_or(v8, 0x000F000Fu, magic) | ((t8 & 0x00010001u) << 4));
+                    const f16x2 b2 = bits2(and_or(v, 0x00F000F0u, magic) | ((t & 0x00020002u) << 7));
+                    const f16x2 b3 = bits2(and_or(v8, 0x00F000F0u, magic) | ((t8 & 0x00020002u) << 7));
+                    p.lo[h] = cat(fma2(b0, s0, q0), fma2(b1, s0, q0), fma2(b2, s1, q1), fma2(b3, s1, q1));
+                }
+            }
+            // mins of sub-blocks 2w, 2w + 1 (w uniform): bytes 2w, 2w + 1 of the 8, each for both its 16-groups
+            const uint32_t mw = and_or(u >> (w < 2 ? 0 : 4), w < 2 ? 0u : 0x0F0F0F0Fu,
+                                       (z >> (w < 2 ? 0 : 2)) & (w < 2 ? 0x3F3F3F3Fu : 0x30303030u));
+            const uint32_t odd = (w & 1) ? 0x00020002u : 0u;
+            const f16x2 ma = bits2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04000400u + odd)) + splat2(-1024.0f);
+            const f16x2 mb = bits2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04010401u + odd)) + splat2(-1024.0f);
+            p.m[0] = f16x4{ma[0], ma[1], mb[0], mb[1]};
+            p.d = h2f(x);
+            p.dmin = -h2f(x >> 16);
+        }
+    };
+
+    float acc[2][CT][4], accm[CT][4];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[0][ct][j] = acc[1][ct][j] = accm[ct][j] = 0.0f;
+    KqCopier<T, CT> copier(a, (uint32_t)(uintptr_t)gm_lds, r0, ct0, wave, lane);
+#pragma unroll 1
+    for (int s = 0; s < S::RING - 1; s++)
+        if (s < nb) copier.issue();
+
+    KqRaw<T> k;
+    f16x8 xb[2][CT];
+    float dx;
+    u32x2 bs;
+    auto read = [&](int stage) {
+        const uint8_t *st = gm_lds + stage * S::BYTES, *W = st + rt * S::WB;
+        // the step's operands: row li's codes of lane slots w, w + 4 and its record; dx and the group sums of column
+        // 16 g + li (the outer products' four column tiles)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const uint8_t *cw = W + k4 * S::TB + h * 256 + (w * 4 + r4) * 16; // the row's qa run of lane slot w + 4h
+            if constexpr (Q6) {
+                const u32x2 x = *reinterpret_cast<const u32x2 *>(cw + 8 * (g >> 1));
+                k.c[2 * h] = x[0];
+                k.c[2 * h + 1] = x[1];
+                k.c[4 + h] = *reinterpret_cast<const uint32_t *>(W + k4 * S::TB + 512 + (w * 4 + r4) * 16 + h * 8 + 4 * (g >> 1));
+            } else {
+                k.c[h] = *reinterpret_cast<const uint32_t *>(cw + 4 * g);
+                if constexpr (T == AQ_TYPE_Q5_K)
+                    k.c[2 + h] = *reinterpret_cast<const uint32_t *>(W + k4 * S::TB + 512 + (w * 4 + r4) * 8 + h * 4);
+            }
+        }
+        k.rec = *reinterpret_cast<const u32x4 *>(W + k4 * S::TB + 512 + S::QB + r4 * 16);
+        if constexpr (Q6) k.d6 = *reinterpret_cast<const uint16_t *>(W + 4 * S::TB + 2 * li);
+        const uint8_t *gm = st + S::GM + g * ACT_GM; // (past the last column tile: whatever is there, not used)
+        dx = *reinterpret_cast<const float *>(gm + 512 + 4 * li);
+        if constexpr (Q6) { // groups 2w, 2w + 1 and 2w + 8, 2w + 9
+            bs[0] = *reinterpret_cast<const uint32_t *>(gm + 32 * li + 4 * w);
+            bs[1] = *reinterpret_cast<const uint32_t *>(gm + 32 * li + 4 * w + 16);
+        } else { // groups 4w .. 4w + 3: sub-blocks 2w, 2w + 1
+            bs = *reinterpret_cast<const u32x2 *>(gm + 32 * li + 8 * w);
+        }
+        // lane slots w and w + 4 are slots 2w and 2w + 1
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++)
+                xb[h][ct] = *reinterpret_cast<const f16x8 *>(st + S::XB + (((2 * w + h) * CT + ct) * 64 + lane) * 16);
+    };
+
+    // A step's products go to the matrix cores from registers; while they run the next stage's copies are met and its
+    // operands read from the LDS, whose latency and bandwidth then hide behind the step's f32 chains.
+    if (S::RING - 1 <= nb) wait_vm_barrier<(S::RING - 2) * S::NDMA>();
+    else wait_vm_barrier<0>();
+    read(0);
+    KqOps ops;
+    unpack(ops, k);
+    int rd = 1; // the next stage to read
+    for (int sb = 0; sb < nb; sb++) {
+        const f16x4 bsv = __builtin_bit_cast(f16x4, bs);
+        f32x16 dd, dmn, pm, off[2];
+        dd = __builtin_amdgcn_mfma_f32_16x16x1f32(ops.d, dx, f32x16{}, 0, 0, 0);
+        if constexpr (Q6) {
+            off[0] = __builtin_amdgcn_mfma_f32_16x16x4f16(ops.m[0], bsv, f32x16{}, 0, 0, 0);
+            off[1] = __builtin_amdgcn_mfma_f32_16x16x4f16(ops.m[1], bsv, f32x16{}, 0, 0, 0);
+        } else {
+            dmn = __builtin_amdgcn_mfma_f32_16x16x1f32(ops.dmin, dx, f32x16{}, 0, 0, 0);
+            pm = __builtin_amdgcn_mfma_f32_16x16x4f16(ops.m[0], bsv, f32x16{}, 0, 0, 0);
+        }
+        f32x4 sl[2][CT], sh4[Q6 ? 2 : 1][Q6 ? CT : 1];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++) {
+                sl[h][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ops.lo[h], xb[h][ct], f32x4{}, 0, 0, 0);
+                if constexpr (Q6) {
+                    const f32x4 o = f32x4{off[h][4 * ct], off[h][4 * ct + 1], off[h][4 * ct + 2], off[h][4 * ct + 3]};
+                    sh4[h][ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ops.hi[h], xb[h][ct], o, 0, 0, 0);
+                }
+            }
+        __builtin_amdgcn_sched_barrier(0);
+        if (sb + 1 < nb) {
+            // stage sb + 1 has landed, and every wave has read stage sb
+            if (sb + S::RING - 1 < nb) wait_vm_barrier<(S::RING - 3) * S::NDMA>();
+            else wait_vm_barrier<0>();
+            if (sb + S::RING - 1 < nb) copier.issue();
+            read(rd);
+            rd = rd + 1 == S::RING ? 0 : rd + 1;
+        }
+        // the f32 chains (kdot.rs:37-140), in super-block order
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float d = dd[4 * ct + j];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    float v = sl[h][ct][j];
+                    if constexpr (Q6) v = __builtin_fmaf(16.0f, sh4[h][ct][j], v); // the exact integer, rounded once
+                    acc[h][ct][j] += d * v;
+                }
+                if constexpr (!Q6) accm[ct][j] += dmn[4 * ct + j] * pm[4 * ct + j];
+            }
+
+        unpack(ops, k);
+    }
+
+    // reduce8 / reduce4 over the waves' lanes: ((l0 + l4) + (l2 + l6)) + ((l1 + l5) + (l3 + l7)), (m0 + m2) + (m1 + m3).
+    // The partials take the ring's place: every copy has landed and been read.
+    __syncthreads();
+    float *part = reinterpret_cast<float *>(gm_lds) + rt * 8 * CT * 256; // [wave][ct][j][lane], then the min lanes
+    float *partm = part + 4 * CT * 256;
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int e = ((w * CT + ct) * 4 + j) * 64 + lane;
+            part[e] = acc[0][ct][j] + acc[1][ct][j];
+            if constexpr (!Q6) partm[e] = accm[ct][j];
+        }
+    __syncthreads();
+    if (w >= CT) return; // wave w finishes column tile w
+    const int col = c0 + 16 * w + li;
+    if (col >= a.ncols) return;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int orow = r0 + 16 * rt + 4 * g + j;
+        if (orow >= a.rows) continue;
+        const int e = (w * 4 + j) * 64 + lane, q = CT * 256;
+        float v = (part[e] + part[2 * q + e]) + (part[q + e] + part[3 * q + e]);
+        if constexpr (!Q6) v = v + ((partm[e] + partm[2 * q + e]) + (partm[q + e] + partm[3 * q + e]));
+        const size_t o = (size_t)col * a.rows + orow;
+        a.y[o] = a.resid ? a.resid[o] + v : v;
     }
 }
 
-// K-quant x Q8_K: a work-group owns 16 rows x 64 columns, wave w the 16 x 16 tile of columns c0 + 16w; lane
-// (li = lane & 15, g = lane >> 4) feeds weight row li / column li into the products (k-group g = sub-blocks 2g,
-// 2g + 1 of each lane slot) and owns the outputs of rows 4g .. 4g + 3 in column li.
-template <int T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) kq_gemm_kernel(GemmArgs a) {
-    using S = KqStage<T>;
-    constexpr int ND = T == AQ_TYPE_Q4_K ? 2 : (T == AQ_TYPE_Q5_K ? 3 : 4); // digits
-    constexpr int BASE = T == AQ_TYPE_Q4_K ? 8 : (T == AQ_TYPE_Q5_K ? 4 : 5);
+template <int T, int CT>
+constexpr size_t kq_lds() {
+    constexpr size_t a = (size_t)KqStage<T, CT>::BYTES * KqStage<T, CT>::RING, b = (size_t)KqStage<T, 1>::BYTES * KqStage<T, 1>::RING;
+    return a > b ? a : b;
+}
+
+template <int T, int CT>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) kq_gemm_kernel(GemmArgs a) {
     extern __shared__ __align__(16) uint8_t gm_lds[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, li = lane & 15, k4 = li >> 2, r4 = li & 3;
-    const int r0 = (int)blockIdx.x * 16;
-    const int c0w = (int)blockIdx.y * 64 + wave * 16;
-    const bool live = c0w < a.ncols; // a wave past the last column copies and waits but computes nothing
-    const int nb = a.nb;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)gm_lds;
-
-    float acc[4][8], accm[4][4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-#pragma unroll
-        for (int l = 0; l < 8; l++) acc[j][l] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) accm[j][i] = 0.0f;
-    }
-#pragma unroll
-    for (int s = 0; s < GEMM_STAGES - 1; s++)
-        if (s < nb) kq_issue<T>(a, lds0 + (uint32_t)(s * S::BYTES), (size_t)s, r0, c0w, wave, lane);
-
-    for (int sb = 0; sb < nb; sb++) {
-        if (sb + GEMM_STAGES - 2 < nb) wait_vm_barrier<(GEMM_STAGES - 2) * S::NDMA>();
-        else wait_vm_barrier<0>();
-        if (sb + GEMM_STAGES - 1 < nb)
-            kq_issue<T>(a, lds0 + (uint32_t)(((sb + GEMM_STAGES - 1) % GEMM_STAGES) * S::BYTES),
-                        (size_t)(sb + GEMM_STAGES - 1), r0, c0w, wave, lane);
-        if (!live) continue;
-        const uint8_t *W = gm_lds + (sb % GEMM_STAGES) * S::BYTES;
-        const uint8_t *X = W + S::WB + wave * S::XB;
-        const uint8_t *SC = W + (S::W_UNITS - 16) * 16;
-
-        // every LDS operand of the step, read up front: the weight codes of row li (lane slots 0..7), the column's
-        // activation codes, the scale records of row li and of the output rows 4g .. 4g + 3, dx and the sums
-        uint32_t wa[8], wb[8], wh[8];
-        uint64_t bx[8];
-#pragma unroll
-        for (int l = 0; l < 8; l++) {
-            const int h = l >> 2, p = l & 3;
-            const int cq = h * 16 + p * 4 + r4; // the lane's qa chunk in its row tile
-            if constexpr (T == AQ_TYPE_Q6_K) {
-                const uint2 w = *reinterpret_cast<const uint2 *>(W + (cq * 4 + k4) * 16 + 8 * (g >> 1));
-                wa[l] = w.x;
-                wb[l] = w.y;
-                wh[l] = *reinterpret_cast<const uint32_t *>(W + 2048 + ((p * 4 + r4) * 4 + k4) * 16 + h * 8 + 4 * (g >> 1));
-            } else {
-                wa[l] = *reinterpret_cast<const uint32_t *>(W + (cq * 4 + k4) * 16 + 4 * g);
-                if constexpr (T == AQ_TYPE_Q5_K) {
-                    const int e = p * 4 + r4;
-                    wh[l] = *reinterpret_cast<const uint32_t *>(W + 2048 + ((e >> 1) * 4 + k4) * 16 + (e & 1) * 8 + h * 4);
-                }
-            }
-            bx[l] = *reinterpret_cast<const uint64_t *>(X + ((lane_slot(l) * 2 + (g >> 1)) * 16 + li) * 16 + 8 * (g & 1));
-        }
-        const uint4 sa = *reinterpret_cast<const uint4 *>(SC + li * 16);
-        uint4 se[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) se[j] = *reinterpret_cast<const uint4 *>(SC + (4 * g + j) * 16);
-        const float dx = *reinterpret_cast<const float *>(X + 4096 + 4 * li);
-        uint4 xs0, xs1;
-        uint2 d6;
-        if constexpr (T == AQ_TYPE_Q6_K) {
-            d6 = *reinterpret_cast<const uint2 *>(W + S::W_UNITS * 16 + 8 * g);
-            xs0 = *reinterpret_cast<const uint4 *>(X + 4160 + 32 * li);
-            xs1 = *reinterpret_cast<const uint4 *>(X + 4160 + 32 * li + 16);
-        } else {
-            xs0 = *reinterpret_cast<const uint4 *>(X + 4160 + 16 * li);
-        }
-
-        // the weight operand's scales: Q4_K / Q5_K as digits of the scales of sub-blocks 2g and 2g + 1; Q6_K as f16
-        // factor pairs of its group scales sc = 16 hi + lo (lo in 0..15, hi in -8..7): (1024 + q) * f - 1024 * f =
-        // q * f, exact (|.| <= 945). Group scale k of the word: 0 = sub-block 2g lanes 0-3, 1 = lanes 4-7, 2 and 3
-        // the same for sub-block 2g + 1.
-        int dga[ND], dgb[ND], dgc[ND], dgd[ND];
-        uint32_t flo[4], clo[4], fhi[4], chi[4];
-        if constexpr (T == AQ_TYPE_Q6_K) {
-            const uint32_t sw = g == 0 ? sa.x : g == 1 ? sa.y : g == 2 ? sa.z : sa.w;
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const int sc = (int8_t)(sw >> (8 * k)), lo = sc & 15, hi = sc >> 4;
-                flo[k] = h2bits((float)lo, (float)lo);
-                clo[k] = h2bits((float)(-1024 * lo), (float)(-1024 * lo));
-                fhi[k] = h2bits((float)hi, (float)hi);
-                chi[k] = h2bits((float)(-1024 * hi), (float)(-1024 * hi));
-            }
-        } else {
-            // 6-bit scales of sub-blocks 2g, 2g + 1 (quant.rs:45-51): bytes 2g, 2g + 1 of the low or high word
-            const uint32_t sc_lo = sa.y & 0x3F3F3F3Fu;
-            const uint32_t sc_hi = (sa.w & 0x0F0F0F0Fu) | ((sa.y >> 2) & 0x30303030u);
-            const uint32_t scw = g < 2 ? sc_lo : sc_hi;
-            const int sca = (int)((scw >> (16 * (g & 1))) & 0xFF), scb = (int)((scw >> (16 * (g & 1) + 8)) & 0xFF);
-            constexpr int BB = T == AQ_TYPE_Q4_K ? 3 : 2;
-#pragma unroll
-            for (int i = 0; i < ND; i++) {
-                dga[i] = dgc[i] = (sca >> (BB * i)) & ((1 << BB) - 1);
-                dgb[i] = dgd[i] = (scb >> (BB * i)) & ((1 << BB) - 1);
-            }
-        }
-
-        // the codes of sub-blocks 2g (lo) and 2g + 1 (hi) per lane slot, as unsigned bytes
-        uint32_t lo[8], hi[8];
-#pragma unroll
-        for (int l = 0; l < 8; l++) {
-            if constexpr (T == AQ_TYPE_Q6_K) {
-                const int sh = 4 * (g & 1);
-                lo[l] = ((wa[l] >> sh) & 0x0F0F0F0Fu) | (((wh[l] >> sh) & 0x03030303u) << 4);
-                hi[l] = ((wb[l] >> sh) & 0x0F0F0F0Fu) | (((wh[l] >> (sh + 2)) & 0x03030303u) << 4);
-            } else {
-                lo[l] = wa[l] & 0x0F0F0F0Fu;
-                hi[l] = (wa[l] >> 4) & 0x0F0F0F0Fu;
-                if constexpr (T == AQ_TYPE_Q5_K) {
-                    lo[l] |= ((wh[l] >> (2 * g)) & 0x01010101u) << 4;
-                    hi[l] |= ((wh[l] >> (2 * g + 1)) & 0x01010101u) << 4;
-                }
-            }
-        }
-
-        // the exact lane sums of the tile: c[l][j] = lane l's sum for output row 4g + j of this lane's column.
-        // Q4_K / Q5_K: int8 products digit by digit over all eight lane slots (eight independent products in flight).
-        // Q6_K: two f16 products per lane slot (the lo and hi scale parts; each sum exact in f32, |.| < 2^22), taken
-        // to i32 and combined there as 16 hi + lo, before the reference's -32 group-sum term (kdot.rs:97-140).
-        v4i c[8];
-        if constexpr (T == AQ_TYPE_Q6_K) {
-#pragma unroll
-            for (int l = 0; l < 8; l++) {
-                const int ka = l < 4 ? 0 : 1, kb = l < 4 ? 2 : 3;
-                const uint32_t la = magic_pair(lo[l], 0), lb = magic_pair(lo[l], 1);
-                const uint32_t ha = magic_pair(hi[l], 0), hb = magic_pair(hi[l], 1);
-                const f16x8 alo = __builtin_bit_cast(
-                    f16x8, uint4{h2fma(la, flo[ka], clo[ka]), h2fma(lb, flo[ka], clo[ka]), h2fma(ha, flo[kb], clo[kb]),
-                                 h2fma(hb, flo[kb], clo[kb])});
-                const f16x8 ahi = __builtin_bit_cast(
-                    f16x8, uint4{h2fma(la, fhi[ka], chi[ka]), h2fma(lb, fhi[ka], chi[ka]), h2fma(ha, fhi[kb], chi[kb]),
-                                 h2fma(hb, fhi[kb], chi[kb])});
-                const f16x8 b = codes_f16(bx[l]);
-                const f32x4 dl = mma_f16(alo, b), dh = mma_f16(ahi, b);
-#pragma unroll
-                for (int e = 0; e < 4; e++) c[l][e] = 16 * (int)dh[e] + (int)dl[e];
-            }
-        } else {
-#pragma unroll
-            for (int i = ND - 1; i >= 0; i--) {
-#pragma unroll
-                for (int l = 0; l < 8; l++) {
-                    const int *da = l < 4 ? dga : dgc, *db = l < 4 ? dgb : dgd;
-                    const uint32_t alo = mul_bytes(lo[l], (uint32_t)da[i]), ahi = mul_bytes(hi[l], (uint32_t)db[i]);
-                    v4i cin = {0, 0, 0, 0};
-                    if (i < ND - 1) {
-#pragma unroll
-                        for (int e = 0; e < 4; e++) cin[e] = c[l][e] * BASE;
-                    }
-                    c[l] = mma(pack2(alo, ahi), bx[l], cin);
-                }
-            }
-        }
-
-        // the f32 chains of the lane's four outputs (kdot.rs:37-140), in super-block order
-        if constexpr (T == AQ_TYPE_Q6_K) {
-            const uint32_t bsw[8] = {xs0.x, xs0.y, xs0.z, xs0.w, xs1.x, xs1.y, xs1.z, xs1.w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t sw[4] = {se[j].x, se[j].y, se[j].z, se[j].w};
-                const float d = dx * h2f((j < 2 ? d6.x : d6.y) >> (16 * (j & 1)));
-#pragma unroll
-                for (int l = 0; l < 8; l++) {
-                    // kdot.rs:125-129: lane l less 32 * (bs[2l] sc[2l] + bs[2l + 1] sc[2l + 1])
-                    const int off = sdot2(bsw[l], i8pair(sw[l >> 1], sw[l >> 1] << 8, 2 * (l & 1)));
-                    acc[j][l] += d * (float)(c[l][j] - 32 * off);
-                }
-            }
-        } else {
-            const uint32_t q8w[4] = {xs0.x, xs0.y, xs0.z, xs0.w};
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float d = dx * h2f(se[j].x), dmin = -dx * h2f(se[j].x >> 16);
-                // the 8 mins as bytes (quant.rs:45-51): sub-blocks 0..3 from bytes 4..7, 4..7 from bytes 8..11 + 4..7
-                const uint32_t mlo = se[j].z & 0x3F3F3F3Fu;
-                const uint32_t mhi = ((se[j].w >> 4) & 0x0F0F0F0Fu) | ((se[j].z >> 2) & 0x30303030u);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const uint32_t m2 = __builtin_amdgcn_perm(0u, i < 2 ? mlo : mhi, (i & 1) ? 0x0C030C02u : 0x0C010C00u);
-                    accm[j][i] += dmin * (float)sdot2(m2, q8w[i]); // m[2i] q8s[2i] + m[2i+1] q8s[2i+1]
-                }
-#pragma unroll
-                for (int l = 0; l < 8; l++) acc[j][l] += d * (float)c[l][j];
-            }
-        }
-    }
-
-    const int ocol = c0w + li;
-    if (live && ocol < a.ncols) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int row = r0 + 4 * g + j;
-            if (row >= a.rows) continue;
-            const float *l8 = acc[j];
-            float v = ((l8[0] + l8[4]) + (l8[2] + l8[6])) + ((l8[1] + l8[5]) + (l8[3] + l8[7])); // reduce8
-            if constexpr (T != AQ_TYPE_Q6_K) {
-                const float *m4 = accm[j];
-                v = v + ((m4[0] + m4[2]) + (m4[1] + m4[3])); // reduce4
-            }
-            const size_t o = (size_t)ocol * a.rows + row;
-            a.y[o] = a.resid ? a.resid[o] + v : v;
-        }
-    }
+    const int b = (int)blockIdx.x, k = b - a.nfull;
+    if (CT == 1 || k < 0) kq_gemm_body<T, CT>(a, gm_lds, 32 * b, 0);
+    else kq_gemm_body<T, 1>(a, gm_lds, 32 * (a.nfull + k / CT), k % CT);
 }
 
 // One step of a Q8_0 / Q4_0 work-group = 8 blocks (256 elements), in 16-byte units: codes unit q * 16 + i = byte
@@ -531,6 +581,36 @@ int launch_staged(K kernel, int bytes, const GemmArgs &ga, hipStream_t stream, c
     return hipGetLastError() == hipSuccess ? 0 : fail(AQ_EHIP, what);
 }
 
+template <int T, int CT>
+int launch_kq_ct(GemmArgs ga, hipStream_t stream) {
+    static std::atomic<uint64_t> raised{0}; // per device: the ring's dynamic LDS allowed
+    int dev = 0;
+    AQ_HIP(hipGetDevice(&dev));
+    const size_t lds = kq_lds<T, CT>();
+    if (!(raised.load() & (1ull << (dev & 63)))) {
+        AQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kq_gemm_kernel<T, CT>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        raised.fetch_or(1ull << (dev & 63));
+    }
+    // A last pass over the CUs whose column tiles fit one pass runs one column tile per work-group (a step of one tile
+    // costs 0.55 of a step of four): the 544 work-groups of 17408 rows are 2.1 passes of 256.
+    const int n = (ga.rows + 31) / 32, over = n % GEMM_CUS;
+    ga.nfull = CT > 2 && n > GEMM_CUS && over * CT <= GEMM_CUS ? n - over : n;
+    const unsigned grid = (unsigned)(ga.nfull + (n - ga.nfull) * CT);
+    hipLaunchKernelGGL((kq_gemm_kernel<T, CT>), dim3(grid), dim3(512), lds, stream, ga);
+    return hipGetLastError() == hipSuccess ? 0 : fail(AQ_EHIP, "kq_gemm launch");
+}
+
+template <int T>
+int launch_kq_gemm(const GemmArgs &ga, hipStream_t stream) {
+    switch ((ga.ncols + 15) / 16) {
+    case 1: return launch_kq_ct<T, 1>(ga, stream);
+    case 2: return launch_kq_ct<T, 2>(ga, stream);
+    case 3: return launch_kq_ct<T, 3>(ga, stream);
+    default: return launch_kq_ct<T, 4>(ga, stream);
+    }
+}
+
 } // namespace
 
 int launch_gemm(const Weight &w, const Act &x, size_t ncols, float *y, const float *resid, hipStream_t stream) {
@@ -550,17 +630,15 @@ int launch_gemm(const Weight &w, const Act &x, size_t ncols, float *y, const flo
     ga.resid = resid;
     if (is_kquant(w.type)) {
         AQ_REQUIRE(w.cols % 256 == 0, "gemm: K-quant columns must be a multiple of 256");
-        ga.xq = x.qs;
-        ga.xd = x.d;
-        ga.xbs = x.bs;
-        ga.xq8s = x.q8s;
+        AQ_REQUIRE(x.gh && x.gm && x.gcap >= ncols && x.gcol == 0, "gemm: the activation has no many-column form");
+        AQ_REQUIRE(ncols <= 64, "gemm: at most 64 columns");
+        ga.gh = x.gh;
+        ga.gm = x.gm;
+        ga.gcap = (uint32_t)x.gcap;
         switch (w.type) {
-        case AQ_TYPE_Q4_K:
-            return launch_staged(kq_gemm_kernel<AQ_TYPE_Q4_K>, KqStage<AQ_TYPE_Q4_K>::BYTES, ga, stream, "kq_gemm launch");
-        case AQ_TYPE_Q5_K:
-            return launch_staged(kq_gemm_kernel<AQ_TYPE_Q5_K>, KqStage<AQ_TYPE_Q5_K>::BYTES, ga, stream, "kq_gemm launch");
-        default:
-            return launch_staged(kq_gemm_kernel<AQ_TYPE_Q6_K>, KqStage<AQ_TYPE_Q6_K>::BYTES, ga, stream, "kq_gemm launch");
+        case AQ_TYPE_Q4_K: return launch_kq_gemm<AQ_TYPE_Q4_K>(ga, stream);
+        case AQ_TYPE_Q5_K: return launch_kq_gemm<AQ_TYPE_Q5_K>(ga, stream);
+        default: return launch_kq_gemm<AQ_TYPE_Q6_K>(ga, stream);
         }
     }
     AQ_REQUIRE(w.type == AQ_TYPE_Q8_0 || w.type == AQ_TYPE_Q4_0, "gemm: weight type");

@@ -447,6 +447,14 @@ Act col_view(const Act &a, size_t col) {
     v.d0 = a.d0 + col * a.nb32;
     v.h0 = a.h0 + col * a.nb32;
     v.s0 = a.s0 + col * a.nb32;
+    v.gcol = a.gcol + col;
+    return v;
+}
+
+// The activation as a pass of t rows writes it: the many-column form only where the many-column products read it.
+Act act_for(const Act &a, size_t t) {
+    Act v = a;
+    if (t <= (size_t)MAX_ROWS) v.gh = nullptr;
     return v;
 }
 
@@ -499,8 +507,9 @@ struct Needs {
 int norm_into(aq_state *s, const float *x, size_t x_stride, const float *norm_w, size_t n, size_t t, Act &act,
               size_t col0, size_t elem_off, const Needs &nd, float *also_f32 = nullptr) {
     const float eps = s->m->cfg.rms_eps;
+    const Act dst = act_for(act, t);
     QuantOut q;
-    q.act = &act;
+    q.act = &dst;
     q.col0 = col0;
     q.elem_off = elem_off;
     q.f32 = true;
@@ -518,7 +527,7 @@ int norm_into(aq_state *s, const float *x, size_t x_stride, const float *norm_w,
 // f32 rows already in act.f32 (columns 0..t) -> the quantised form(s).
 int quantize_act(aq_state *s, Act &act, size_t t, const Needs &nd) {
     int rc = 0;
-    if (nd.q8k) rc = launch_q8k_quantize(act, t, act.f32, act.n, s->stream);
+    if (nd.q8k) rc = launch_q8k_quantize(act_for(act, t), t, act.f32, act.n, s->stream);
     if (!rc && nd.q80) rc = launch_q8_0_quantize(act, t, act.f32, act.n, s->stream);
     return rc;
 }
@@ -621,8 +630,9 @@ float *dn_beta_out(aq_state *s, Mode mode, int dn_slot) { return mode == VERIFY 
 // attn_norm of a DeltaNet layer into act_h (f32 + Q8_K) with its gate rows (dn_gates_in_norm), one launch.
 int norm_gates_into(aq_state *s, const DevLayer &L, const float *x, size_t t, Mode mode, int dn_slot) {
     const size_t h = s->m->cfg.hidden;
+    const Act dst = act_for(s->act_h, t);
     QuantOut q;
-    q.act = &s->act_h;
+    q.act = &dst;
     q.kind = QK_Q8K;
     q.f32 = true;
     NormRows fr;
@@ -666,7 +676,8 @@ int mixer(aq_state *s, const DevLayer &L, size_t t, size_t start_pos, KvDev *kv,
         // the o projection reads Q8_K: each head's output row (head_dim 256) is quantised by the attention kernel
         const bool q8k = quant_kind_for(L.o.type) == QK_Q8K && c.head_dim == 256;
         a.out_q8k = q8k ? 1 : 0;
-        a.q8k = s->act_att;
+        const Act att = act_for(s->act_att, t);
+        a.q8k = att;
         a.t = (int)t;
         a.nh = (int)c.n_head;
         a.nkv = (int)c.n_head_kv;
@@ -689,7 +700,7 @@ int mixer(aq_state *s, const DevLayer &L, size_t t, size_t start_pos, KvDev *kv,
             ap.vv = a.vv + r0 * kw;
             ap.q = a.q + r0 * ow;
             ap.out = a.out + r0 * ow;
-            ap.q8k = col_view(s->act_att, r0);
+            ap.q8k = col_view(att, r0);
             ap.start_pos = start_pos + r0;
             ap.base = kv->len;
             ap.t = (int)tr;
@@ -757,8 +768,9 @@ int mlp(aq_state *s, const DevLayer &L, size_t t, float *y_out, const float *res
     float *ys[2] = {s->g, s->u};
     int rc = mm_multi(s, 2, ws, ys, s->act_h, t);
     if (rc) return rc;
+    const Act dst = act_for(s->act_ffn, t);
     QuantOut q;
-    q.act = &s->act_ffn;
+    q.act = &dst;
     q.kind = quant_kind_for(L.down.type);
     if ((rc = launch_swiglu(s->g, s->u, ffn, t, q.kind == QK_NONE ? s->act_ffn.f32 : nullptr, q, s->stream))) return rc;
     return mm(s, L.down, s->act_ffn, t, y_out, resid);

@@ -108,9 +108,15 @@ __device__ __forceinline__ int wave_min_i32(int v) {
 // (q8k.rs:76-114): max = the first element with the largest |x|, iscale = -127/max, q = min(127,
 // round_ties_even(iscale*x)), d = 1/iscale (0 for an all-zero block), bsums per 16, q8s per 32. The largest |x|
 // (a max, order-free) and then its first index (a min over lanes) come from DPP reductions. Writes the block at
-// (qs_blk, *d_out, bs_blk[16], q8s_blk[8]) in the kernels' lane-slot code order.
+// (qs_blk, *d_out, bs_blk[16], q8s_blk[8]) in the kernels' lane-slot code order, and where gh is set the many-column
+// form: this lane's four codes at gh, the block's group sums and d at gb and gd.
+__device__ __forceinline__ uint32_t f16_pair(int a, int b) {
+    typedef _Float16 f16x2_q __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, f16x2_q{(_Float16)(float)a, (_Float16)(float)b});
+}
 __device__ __forceinline__ void q8k_block_wave(const float x[4], int lane, int8_t *qs_blk, float *d_out,
-                                               int16_t *bs_blk, int16_t *q8s_blk) {
+                                               int16_t *bs_blk, int16_t *q8s_blk, uint16_t *gh, uint16_t *gb,
+                                               float *gd) {
     float la = fabsf(x[0]);
 #pragma unroll
     for (int j = 1; j < 4; j++) la = fmaxf(la, fabsf(x[j]));
@@ -131,18 +137,27 @@ __device__ __forceinline__ void q8k_block_wave(const float x[4], int lane, int8_
             const int qi = (int)__builtin_rintf(iscale * x[j]);
             q[j] = qi < 127 ? qi : 127;
         }
-        if (lane == 0) *d_out = 1.0f / iscale;
+        if (lane == 0) {
+            const float d = 1.0f / iscale;
+            *d_out = d;
+            if (gh) *gd = d;
+        }
     } else if (lane == 0) {
         *d_out = 0.0f;
+        if (gh) *gd = 0.0f;
     }
     const int s = lane >> 3, l = lane & 7;
+    if (gh) *reinterpret_cast<uint2 *>(gh) = make_uint2(f16_pair(q[0], q[2]), f16_pair(q[1], q[3]));
     const uint32_t packed = (uint32_t)(uint8_t)q[0] | ((uint32_t)(uint8_t)q[1] << 8) | ((uint32_t)(uint8_t)q[2] << 16) |
                             ((uint32_t)(uint8_t)q[3] << 24);
     *reinterpret_cast<uint32_t *>(qs_blk + lane_slot(l) * 32 + s * 4) = packed;
     int sum = q[0] + q[1] + q[2] + q[3];
     sum += dpp_mov<0xB1>(sum); // quad: the 16 values of a group
     sum += dpp_mov<0x4E>(sum);
-    if ((lane & 3) == 0) bs_blk[lane >> 2] = (int16_t)sum;
+    if ((lane & 3) == 0) {
+        bs_blk[lane >> 2] = (int16_t)sum;
+        if (gh) gb[lane >> 2] = (uint16_t)f16_pair(sum, 0);
+    }
     const int s32 = sum + dpp_mov<0x12C>(sum); // row_ror:12 = lane i + 4: the next quad, a 32-value sub-block
     if ((lane & 7) == 0) q8s_blk[lane >> 3] = (int16_t)s32;
 }
@@ -150,7 +165,15 @@ __device__ __forceinline__ void q8k_block_wave(const float x[4], int lane, int8_
 // Store block `blk` of column `col` of a Q8_K activation.
 __device__ __forceinline__ void q8k_block_store(const Act &a, size_t col, size_t blk, const float x[4], int lane) {
     const size_t m = col * a.nb + blk;
-    q8k_block_wave(x, lane, a.qs + col * a.n + blk * 256, a.d + m, a.bs + m * 16, a.q8s + m * 8);
+    if (a.gh) { // lane 8 s + l holds lane l's elements of sub-block s
+        const int s = lane >> 3, c = (int)((a.gcol + col) % 16);
+        uint16_t *gh = a.gh + act_gh(a.gcap, blk, lane_slot(lane & 7), a.gcol + col, s >> 1) + 4 * (s & 1);
+        uint8_t *gm = a.gm + act_gm(a.gcap, blk, a.gcol + col);
+        q8k_block_wave(x, lane, a.qs + col * a.n + blk * 256, a.d + m, a.bs + m * 16, a.q8s + m * 8, gh,
+                       reinterpret_cast<uint16_t *>(gm + 32 * c), reinterpret_cast<float *>(gm + 512 + 4 * c));
+        return;
+    }
+    q8k_block_wave(x, lane, a.qs + col * a.n + blk * 256, a.d + m, a.bs + m * 16, a.q8s + m * 8, nullptr, nullptr, nullptr);
 }
 
 // Max / sum of ints over each 32-lane half of a wave (order-free, so exact): every lane gets its half's value. The

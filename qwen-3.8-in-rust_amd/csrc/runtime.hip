@@ -138,7 +138,10 @@ int alloc_act(Act &a, size_t n, size_t ncols, int device) {
     const size_t f = align256(ncols * n * 4), q = align256(ncols * n), d = align256(ncols * a.nb * 4 + 4),
                  bs = align256(ncols * a.nb * 32 + 4), q8s = align256(ncols * a.nb * 16 + 4), q0 = align256(ncols * n),
                  d0 = align256(ncols * a.nb32 * 4), h0 = align256(ncols * a.nb32 * 2), s0 = align256(ncols * a.nb32 * 4);
-    const size_t total = f + q + d + bs + q8s + q0 + d0 + h0 + s0;
+    // the many-column form, where the buffer can hold more columns than the verify kernels take
+    const size_t gcap = ncols > 8 ? (ncols + 15) / 16 * 16 : 0;
+    const size_t gh = align256(gcap * a.nb * 512), gm = align256(gcap / 16 * a.nb * ACT_GM);
+    const size_t total = f + q + d + bs + q8s + q0 + d0 + h0 + s0 + gh + gm;
     void *p = nullptr;
     if (dev_malloc(&p, total) != hipSuccess) return fail(AQ_ENOMEM, "act: hipMalloc");
     if (hipMemset(p, 0, total) != hipSuccess) return fail(AQ_EHIP, "act: hipMemset");
@@ -163,6 +166,12 @@ int alloc_act(Act &a, size_t n, size_t ncols, int device) {
     a.h0 = (uint16_t *)b;
     b += h0;
     a.s0 = (int32_t *)b;
+    b += s0;
+    a.gcap = gcap;
+    if (gcap) {
+        a.gh = (uint16_t *)b;
+        a.gm = b + gh;
+    }
     return 0;
 }
 
