@@ -834,8 +834,9 @@ int mtp_set_rows(aq_state *s, const uint32_t *ids_dev, const float *hs, size_t t
         if (!rc) rc = norm_into(s, hs, h, m->hnorm, h, t, s->act_cat, 0, h, nd);
         return rc;
     }
+    const Act dst = act_for(s->act_cat, t);
     QuantOut q; // both halves in one launch
-    q.act = &s->act_cat;
+    q.act = &dst;
     q.col0 = 0;
     q.elem_off = 0;
     q.f32 = true;
@@ -1083,11 +1084,11 @@ int aq_state_new(aq_model *m, uint32_t spec_k, uint32_t max_pos, aq_state **out)
     AQ_S(alloc_act(s->act_ffn, c.ffn, TP, m->ctx->device));
     AQ_S(alloc_act(s->act_vd, m->vd, TP, m->ctx->device));
     AQ_S(alloc_act(s->act_att, (size_t)c.n_head * c.head_dim, TP, m->ctx->device));
-    AQ_S(alloc_act(s->act_cat, 2 * h, T, m->ctx->device));
+    AQ_S(alloc_act(s->act_cat, 2 * h, TP, m->ctx->device));
     AQ_S(dalloc_t(s, TP * h, &s->xa));
     AQ_S(dalloc_t(s, TP * h, &s->xb));
     AQ_S(dalloc_t(s, TP * h, &s->y));
-    AQ_S(dalloc_t(s, T * h, &s->e));
+    AQ_S(dalloc_t(s, TP * h, &s->e));
     AQ_S(dalloc_t(s, TP * m->cd, &s->mixed));
     AQ_S(dalloc_t(s, TP * m->vd, &s->z));
     AQ_S(dalloc_t(s, TP * nv, &s->a));
@@ -1101,7 +1102,7 @@ int aq_state_new(aq_model *m, uint32_t spec_k, uint32_t max_pos, aq_state **out)
     AQ_S(dalloc_t(s, T * c.vocab, &s->logits));
     AQ_S(dalloc_t(s, T * h, &s->normed));
     AQ_S(dalloc_t(s, (size_t)s->max_pos * h, &s->normed_all));
-    AQ_S(dalloc_t(s, T * h, &s->mtp_hout));
+    AQ_S(dalloc_t(s, TP * h, &s->mtp_hout));
     AQ_S(dalloc_t(s, T, &s->ids));
     AQ_S(dalloc_t(s, T, &s->amax));
     AQ_S(dalloc_t(s, T, &s->drafts));
@@ -1246,8 +1247,8 @@ int aq_spec_prefill(aq_state *s, const uint32_t *ids, size_t n, uint32_t *x_t) {
     if (n > 1) AQ_HIP(hipMemcpyAsync(s->shifted, s->prompt + 1, (n - 1) * 4, hipMemcpyDeviceToDevice, s->stream));
     AQ_HIP(hipMemcpyAsync(s->shifted + (n - 1), s->amax, 4, hipMemcpyDeviceToDevice, s->stream));
     size_t last = 0;
-    for (size_t c0 = 0; c0 < n; c0 += MAX_ROWS) {
-        const size_t tc = n - c0 < (size_t)MAX_ROWS ? n - c0 : (size_t)MAX_ROWS;
+    for (size_t c0 = 0; c0 < n; c0 += PRE_ROWS) { // in the prompt's own chunks: its weights read once per chunk
+        const size_t tc = n - c0 < (size_t)PRE_ROWS ? n - c0 : (size_t)PRE_ROWS;
         AQ_REQUIRE(s->mtp_kv.len + tc <= s->mtp_kv.cap, "aq_spec_prefill: MTP cache full");
         if ((rc = mtp_set_rows(s, s->shifted + c0, s->normed_all + c0 * h, tc))) return rc;
         if ((rc = mtp_rows(s, tc))) return rc;
