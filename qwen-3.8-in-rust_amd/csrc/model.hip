@@ -414,6 +414,7 @@ struct aq_state {
     aq::Act act_h, act_ffn, act_vd, act_att, act_cat;
     float *xa = nullptr, *xb = nullptr, *y = nullptr, *mixed = nullptr, *z = nullptr, *a = nullptr, *b = nullptr;
     float *qg = nullptr, *kk = nullptr, *vv = nullptr, *qr = nullptr, *g = nullptr, *u = nullptr, *e = nullptr;
+    float *dn_pre = nullptr; // a prompt chunk's DeltaNet inputs (dn_chunk_floats)
     float *logits = nullptr, *normed = nullptr, *normed_all = nullptr, *mtp_hout = nullptr;
     float *cos_tab = nullptr, *sin_tab = nullptr;
     uint32_t *ids = nullptr, *amax = nullptr, *drafts = nullptr, *emitted = nullptr, *info = nullptr, *prompt = nullptr,
@@ -750,7 +751,8 @@ int mixer(aq_state *s, const DevLayer &L, size_t t, size_t start_pos, KvDev *kv,
     d.dk = (int)c.dn_head_dim_k;
     d.dv = (int)c.dn_head_dim_v;
     d.kernel = (int)c.dn_conv_kernel;
-    // a prompt chunk (t > 8) runs as 8-row pieces inside the one launch, the state carried from piece to piece
+    d.pre = s->dn_pre;
+    // a prompt chunk (t > 8) writes the state: PLAIN passes only
     AQ_REQUIRE(t <= 8 || mode == PLAIN, "deltanet: more than 8 rows in one verify batch");
     if ((rc = launch_dn_core(d, s->stream))) return rc;
     if (!q80) {
@@ -1090,6 +1092,15 @@ int aq_state_new(aq_model *m, uint32_t spec_k, uint32_t max_pos, aq_state **out)
     AQ_S(dalloc_t(s, TP * h, &s->y));
     AQ_S(dalloc_t(s, TP * h, &s->e));
     AQ_S(dalloc_t(s, TP * m->cd, &s->mixed));
+    {
+        DnArgs d;
+        d.t = (int)TP;
+        d.nk = (int)c.dn_n_k_heads;
+        d.nv = (int)c.dn_n_v_heads;
+        d.dk = (int)c.dn_head_dim_k;
+        d.dv = (int)c.dn_head_dim_v;
+        AQ_S(dalloc_t(s, dn_chunk_floats(d), &s->dn_pre));
+    }
     AQ_S(dalloc_t(s, TP * m->vd, &s->z));
     AQ_S(dalloc_t(s, TP * nv, &s->a));
     AQ_S(dalloc_t(s, TP * nv, &s->b));

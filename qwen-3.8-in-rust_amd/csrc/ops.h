@@ -76,9 +76,15 @@ struct DnArgs {
     int raw = 0;
     const float *rq = nullptr, *rk = nullptr, *rv = nullptr, *rg = nullptr, *rbeta = nullptr;
     const uint32_t *t_dev = nullptr; // multi launch: the row count, read on the device (1..8)
+    float *pre = nullptr; // prompt chunks: dn_chunk_floats of scratch
 };
-// t rows; more than 8 (a prompt chunk: projected gates, no raw mode) run as 8-row pieces inside one launch.
+// t rows, up to 8 in one launch; more (a prompt chunk) by launch_dn_chunk.
 int launch_dn_core(const DnArgs &a, hipStream_t stream);
+// A prompt chunk's rows (deltanet_chunk.hip): projected gates (no raw mode), `pre` set, the state and the conv window
+// written.
+int launch_dn_chunk(const DnArgs &a, hipStream_t stream);
+// Floats of `pre` for t rows.
+size_t dn_chunk_floats(const DnArgs &a);
 // n DnArgs (device array, commit form: saved gates, no output), all with the head shape of `like`: one launch.
 int launch_dn_core_multi(const DnArgs *args_dev, const DnArgs &like, int n, hipStream_t stream);
 

@@ -420,21 +420,13 @@ constexpr int dn_parts() {
     return (4 * DV <= DN_THREADS && DK % 16 == 0) ? 4 : (2 * DV <= DN_THREADS && DK % 8 == 0) ? 2 : 1;
 }
 
-template <int DK, int DV>
-constexpr int dn_kh() { return DK / dn_parts<DK, DV>(); }
-
-// Rows r0 .. r0 + t - 1 (t <= DN_TMAX) of the launch's rows. `s` is the thread's part of the state column: loaded
-// from a.rec when `first`, written back when `last` (and a.write_state), carried in registers between the pieces of
-// one launch otherwise. The conv window of a piece after the first is the three input rows before it. TT > 0: the
-// row count is TT (the input loops run over exactly those rows), else t_in.
-template <int DK, int DV, bool CHUNK = false, int TT = 0>
-__device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const int t_in, float (&s)[dn_kh<DK, DV>()],
-                                             const int r0, const bool first, const bool last) {
+// The launch's t <= DN_TMAX rows. TT > 0: the row count is TT (the input loops run over exactly those rows), else t_in.
+template <int DK, int DV, int TT = 0>
+__device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const int t_in) {
     static_assert(TT >= 0 && TT <= DN_TMAX, "rows per launch");
     constexpr int TM = TT ? TT : DN_TMAX; // the input loops' bound
     const int t = TT ? TT : t_in;
-    // CHUNK: the host admits no raw rows, so that path compiles away
-    const bool raw_ = !CHUNK && a.raw;
+    const bool raw_ = a.raw;
     static_assert(DK <= 256 && DV <= 256 && DN_THREADS >= 448 && DN_TMAX * 2 <= 16, "DeltaNet work-group shape");
     __shared__ float sq[DN_TMAX][DK], sk[DN_TMAX][DK], sv[DN_TMAX][DV], sz[DN_TMAX][DV], so[DN_TMAX][DV];
     __shared__ float rdec[DN_TMAX], rbeta[DN_TMAX], rq[DN_TMAX], rk[DN_TMAX], ro[DN_TMAX];
@@ -448,8 +440,8 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
     const int gr = wave == 5 ? 0 : 1;
     float gv = 0.0f, gsa = 0.0f, gdt = 0.0f;
     if (gate_lane) {
-        gv = raw_ ? (gr == 0 ? a.rg : a.rbeta)[(size_t)(r0 + lane) * a.nv + p]
-                  : (gr == 0 ? a.a : a.b)[(size_t)(r0 + lane) * a.nv + p];
+        gv = raw_ ? (gr == 0 ? a.rg : a.rbeta)[(size_t)lane * a.nv + p]
+                  : (gr == 0 ? a.a : a.b)[(size_t)lane * a.nv + p];
         if (gr == 0 && !raw_) {
             gsa = a.ssm_a[p];
             gdt = a.dt_bias[p];
@@ -462,7 +454,8 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
     const int c = j % DV, h = j / DV;
     const bool has_col = h < H;
     float *srec = a.rec + (size_t)p * DK * DV;
-    if (has_col && first) {
+    float s[KH];
+    if (has_col) {
 #pragma unroll
         for (int k = 0; k < KH; k++) s[k] = srec[(size_t)(h * KH + k) * DV + c];
     }
@@ -471,12 +464,12 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
     if (raw_) {
         for (int e = j; e < t * DK; e += DN_THREADS) {
             const int i = e / DK, c = e % DK;
-            sq[i][c] = a.rq[(size_t)(r0 + i) * kd + kh * DK + c];
-            sk[i][c] = a.rk[(size_t)(r0 + i) * kd + kh * DK + c];
+            sq[i][c] = a.rq[(size_t)i * kd + kh * DK + c];
+            sk[i][c] = a.rk[(size_t)i * kd + kh * DK + c];
         }
         for (int e = j; e < t * DV; e += DN_THREADS) {
             const int i = e / DV, c = e % DV;
-            sv[i][c] = a.rv[(size_t)(r0 + i) * vd + p * DV + c];
+            sv[i][c] = a.rv[(size_t)i * vd + p * DV + c];
         }
     } else {
         // task c: q channel c (c < DK), k channel c - DK, v channel c - 2 DK (conv, conv.rs:11-36), then the
@@ -490,12 +483,12 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
                 float seq[TM + 3];
 #pragma unroll
                 for (int e = 0; e < 3; e++)
-                    seq[e] = first ? a.conv_src[(size_t)ch * 3 + e] : a.mixed[(size_t)(r0 - 3 + e) * cd + ch];
+                    seq[e] = a.conv_src[(size_t)ch * 3 + e];
                 float cw[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) cw[e] = a.conv_w[(size_t)ch * 4 + e];
 #pragma unroll
-                for (int i = 0; i < TM; i++) seq[3 + i] = a.mixed[(size_t)(r0 + (i < t ? i : t - 1)) * cd + ch];
+                for (int i = 0; i < TM; i++) seq[3 + i] = a.mixed[(size_t)(i < t ? i : t - 1) * cd + ch];
                 float *dst = kind == 0 ? &sq[0][cc] : kind == 1 ? &sk[0][cc] : &sv[0][cc];
                 const int dstride = kind == 2 ? DV : DK;
 #pragma unroll
@@ -509,7 +502,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
                         dst[i * dstride] = silu_f(acc);
                     }
                 }
-                if (a.conv_dst && last && (kind == 2 || p == kh)) {
+                if (a.conv_dst && (kind == 2 || p == kh)) {
 #pragma unroll
                     for (int i = 0; i <= TM; i++) // the window after row t - 1: seq[t .. t + 2]
                         if (i == t)
@@ -519,7 +512,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
                 const int cc = c - n_conv;
                 float zr[TM];
 #pragma unroll
-                for (int i = 0; i < TM; i++) zr[i] = a.z[(size_t)(r0 + (i < t ? i : t - 1)) * vd + p * DV + cc];
+                for (int i = 0; i < TM; i++) zr[i] = a.z[(size_t)(i < t ? i : t - 1) * vd + p * DV + cc];
 #pragma unroll
                 for (int i = 0; i < TM; i++)
                     if (i < t) sz[i][cc] = silu_f(zr[i]);
@@ -650,7 +643,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
                 if (hh + 1 < H) {
                     xfer2[c] = ov;
                 } else if (raw_) {
-                    if (a.out) a.out[(size_t)(r0 + i) * vd + p * DV + c] = ov;
+                    if (a.out) a.out[(size_t)i * vd + p * DV + c] = ov;
                 } else {
                     so[i][c] = ov;
                 }
@@ -658,7 +651,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
             if (hh + 1 < H) __syncthreads();
         }
     }
-    if (has_col && a.write_state && last) {
+    if (has_col && a.write_state) {
 #pragma unroll
         for (int k = 0; k < KH; k++) srec[(size_t)(h * KH + k) * DV + c] = s[k];
     }
@@ -690,8 +683,8 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
             const int i = e / DV, jc = e % DV;
             const float w = e == j ? nrm_w : a.ssm_norm[jc];
             const float v = (w * (so[i][jc] * ro[i])) * sz[i][jc];
-            a.out[(size_t)(r0 + i) * vd + p * DV + jc] = v;
-            if (a.out_q80) q8_0_block_half(a.q80, r0 + i, (size_t)p * (DV / 32) + (jc >> 5), v, lane);
+            a.out[(size_t)i * vd + p * DV + jc] = v;
+            if (a.out_q80) q8_0_block_half(a.q80, i, (size_t)p * (DV / 32) + (jc >> 5), v, lane);
         }
     }
 }
@@ -699,21 +692,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
 // TT > 0: a.t == TT rows (the verify's k + 1 and decode's 1 take such an instance), else any row count up to 8
 template <int DK, int DV, int TT>
 __global__ void __launch_bounds__(DN_THREADS) dn_core_kernel(DnArgs a) {
-    float s[dn_kh<DK, DV>()];
-    dn_core_body<DK, DV, false, TT>(a, (int)blockIdx.x, a.t, s, 0, true, true);
-}
-
-// A prompt chunk of more than DN_TMAX rows in one launch (gated_deltanet.rs:197-199 steps the recurrence token by
-// token): pieces of DN_TMAX rows in order, the state column kept in registers from piece to piece and each piece's
-// conv window taken from the three input rows before it.
-template <int DK, int DV>
-__global__ void __launch_bounds__(DN_THREADS) dn_core_chunk_kernel(DnArgs a) {
-    float s[dn_kh<DK, DV>()];
-    for (int r0 = 0; r0 < a.t; r0 += DN_TMAX) {
-        if (r0 > 0) __syncthreads(); // the previous piece's LDS rows are read to the end before they are rewritten
-        const int tp = a.t - r0 < DN_TMAX ? a.t - r0 : DN_TMAX;
-        dn_core_body<DK, DV, true>(a, (int)blockIdx.x, tp, s, r0, r0 == 0, r0 + DN_TMAX >= a.t);
-    }
+    dn_core_body<DK, DV, TT>(a, (int)blockIdx.x, a.t);
 }
 
 // Several layers' heads in one launch (the commit of every DeltaNet layer after a speculative round): work-group
@@ -723,8 +702,7 @@ __global__ void __launch_bounds__(DN_THREADS) dn_core_multi_kernel(const DnArgs 
     const DnArgs &a = args[blockIdx.y];
     const int t = a.t_dev ? (int)*a.t_dev : a.t;
     if (t < 1 || t > DN_TMAX) return; // uniform: a row count the host validates before it is used
-    float s[dn_kh<DK, DV>()];
-    dn_core_body<DK, DV>(a, (int)blockIdx.x, t, s, 0, true, true);
+    dn_core_body<DK, DV>(a, (int)blockIdx.x, t);
 }
 
 // ---------------------------------------------------------------------------------------------- attention
@@ -1188,22 +1166,20 @@ int launch_dn_core(const DnArgs &a, hipStream_t stream) {
     } else {
         AQ_REQUIRE(a.rq && a.rk && a.rv && a.rg && a.rbeta, "deltanet: raw inputs");
     }
-    AQ_REQUIRE(a.t <= DN_TMAX || (!a.raw && a.t <= 4096),
-               "deltanet: more than 8 rows in one launch need the projected gates (no raw mode) and t <= 4096");
     AQ_REQUIRE(a.raw || (a.a && a.b), "deltanet: gate inputs");
     const int threads = DN_THREADS;
     const int key = a.dk * 1000 + a.dv;
     switch (key) {
 #define AQ_DN(K, V)                                                                                           \
     case K * 1000 + V:                                                                                        \
-        if (a.t == 4)                                                                                         \
+        if (a.t > DN_TMAX)                                                                                    \
+            return launch_dn_chunk(a, stream);                                                                \
+        else if (a.t == 4)                                                                                    \
             hipLaunchKernelGGL((dn_core_kernel<K, V, 4>), dim3((unsigned)a.nv), dim3(threads), 0, stream, a);  \
         else if (a.t == 1)                                                                                    \
             hipLaunchKernelGGL((dn_core_kernel<K, V, 1>), dim3((unsigned)a.nv), dim3(threads), 0, stream, a);  \
-        else if (a.t <= DN_TMAX)                                                                              \
-            hipLaunchKernelGGL((dn_core_kernel<K, V, 0>), dim3((unsigned)a.nv), dim3(threads), 0, stream, a);  \
         else                                                                                                  \
-            hipLaunchKernelGGL((dn_core_chunk_kernel<K, V>), dim3((unsigned)a.nv), dim3(threads), 0, stream, a); \
+            hipLaunchKernelGGL((dn_core_kernel<K, V, 0>), dim3((unsigned)a.nv), dim3(threads), 0, stream, a);  \
         break;
         AQ_DN(8, 8) AQ_DN(16, 16) AQ_DN(32, 32) AQ_DN(64, 64) AQ_DN(128, 128) AQ_DN(128, 256) AQ_DN(64, 128)
 #undef AQ_DN
