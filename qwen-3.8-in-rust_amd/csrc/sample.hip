@@ -4,8 +4,9 @@
 //
 // Candidates. A logit and its id form one 64-bit key, (the logit's order bits, descending) << 32 | id, so ascending
 // keys are the reference's order: logit descending, ties by the lower id (sample.rs:196; -0 and +0 are one key).
-// top_k <= 512: every 4096-key chunk of the row is sorted in LDS (bitonic) and keeps its first top_k keys; lists are
-// merged the same way until one remains. Larger top_k or none: the row's keys are radix-sorted whole (hipcub).
+// top_k <= 512: every 4096-key chunk of the row keeps its first top_k keys, in order; lists are merged the same way
+// until one remains. Up to 128 a chunk's first keys are selected by a bound before anything is sorted (topk_few_kernel),
+// past that the chunk is sorted whole in LDS (bitonic). Larger top_k or none: the row's keys are radix-sorted (hipcub).
 //
 // The rest is one 256-thread work-group: elementwise steps in parallel; the reference's sequential f32 sums (the
 // softmax denominator, the renormalisation, top-p's running mass, the draw's running mass, the residual's sum) by
@@ -28,6 +29,8 @@ namespace {
 constexpr int ST = 256;          // sampler work-group
 constexpr int SZ = 4096;         // keys sorted per chunk work-group
 constexpr int KMAX_FAST = 512;   // top_k up to this takes the chunked selection
+constexpr int KMAX_FEW = 128;    // up to this by a bound on each chunk's keys
+constexpr int FEW = 512;         // keys at or under the bound that are ranked (more: the whole chunk is sorted)
 constexpr int ROWS_MAX = 17;     // rows per call (k + 1 for k <= 16)
 enum { OP_PROCESS = 0, OP_DRAW = 1, OP_SAMPLE = 2, OP_ACCEPT = 3, OP_DRAFT = 4, OP_ROUND = 5, OP_GREEDY_SET = 6 };
 
@@ -76,6 +79,102 @@ __global__ void __launch_bounds__(ST) topk_chunk_kernel(const float *lg, size_t 
     __syncthreads();
     bitonic_sz(s);
     for (int j = threadIdx.x; j < K; j += ST) out[(size_t)r * out_stride + (size_t)c * K + j] = s[j];
+}
+
+// How many of n keys in LDS are less than key (every lane reads the same keys: two per broadcast load).
+__device__ __forceinline__ int rank_of(uint64_t key, const uint64_t *s, int n) {
+    int less = 0;
+#pragma unroll 8
+    for (int i = 0; i < n; i += 2) { // (s[n] may be read: the array is longer)
+        const ulonglong2 p = *reinterpret_cast<const ulonglong2 *>(s + i);
+        less += p.x < key ? 1 : 0;
+        less += i + 1 < n && p.y < key ? 1 : 0;
+    }
+    return less;
+}
+
+// The same for K <= KMAX_FEW. Each thread holds 16 of the chunk's keys; the K-th smallest of the threads' smallest keys
+// bounds the chunk's K-th smallest (K distinct keys are at or under it), so the first K are among the keys at or under
+// the bound - little more than K when the row is in no particular order - and only those are put in order. Keys are
+// distinct, so a key's place is the number of smaller ones, counted by its thread without a barrier. Sorting all 4096
+// took 100 us per launch (78 steps of 8 exchanges per thread, each with a barrier); this takes 8 at 40 of 248,320.
+__global__ void __launch_bounds__(ST) topk_few_kernel(const float *lg, size_t lg_stride, int vocab, const uint64_t *in,
+                                                      size_t in_stride, int in_count, int K, uint64_t *out,
+                                                      size_t out_stride) {
+    __shared__ __attribute__((aligned(16))) uint64_t s[SZ];
+    __shared__ uint64_t s_bound;
+    __shared__ int s_n;
+    const int c = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
+    constexpr int PER = SZ / ST;
+    uint64_t key[PER], least = ~0ull;
+    // Thread tid's u-th key: 256 in a row per load, turned by 37 each time, so that the heads of the sorted lists a later
+    // launch reads (every K keys, K often dividing 256) fall to different threads.
+    auto key_at = [&](int u) { return c * SZ + u * ST + ((tid + 37 * u) & (ST - 1)); };
+    if (in == nullptr) {
+        float v[PER];
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const int g = key_at(u);
+            v[u] = lg[(size_t)r * lg_stride + min(g, vocab - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const int g = key_at(u);
+            key[u] = g < vocab ? make_key(v[u], (uint32_t)g) : ~0ull;
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < PER; u++) key[u] = in[(size_t)r * in_stride + min(key_at(u), in_count - 1)];
+#pragma unroll
+        for (int u = 0; u < PER; u++)
+            if (key_at(u) >= in_count) key[u] = ~0ull;
+    }
+#pragma unroll
+    for (int u = 0; u < PER; u++) least = key[u] < least ? key[u] : least;
+    s[tid] = least;
+    if (tid == 0) {
+        s_n = 0;
+        s_bound = ~0ull; // fewer than K threads have a key: all of them
+    }
+    __syncthreads();
+    if (least != ~0ull && rank_of(least, s, ST) == K - 1) s_bound = least;
+    __syncthreads();
+    const uint64_t bound = s_bound;
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+        if (key[u] <= bound && key[u] != ~0ull) { // (~0: no key)
+            const int at = atomicAdd(&s_n, 1);
+            if (at < FEW) s[at] = key[u];
+        }
+    __syncthreads();
+    const int n = s_n;
+    uint64_t *dst = out + (size_t)r * out_stride + (size_t)c * K;
+    if (n <= FEW) {
+        for (int i = tid; i < n; i += ST) {
+            const uint64_t mine = s[i];
+            const int at = rank_of(mine, s, n);
+            if (at < K) dst[at] = mine;
+        }
+        for (int i = n + tid; i < K; i += ST) dst[i] = ~0ull;
+    } else { // an ordered row: sort the chunk
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < PER; u++) s[u * ST + tid] = key[u];
+        __syncthreads();
+        bitonic_sz(s);
+        for (int i = tid; i < K; i += ST) dst[i] = s[i];
+    }
+}
+
+// `write_dense` (sample.rs:259-265): zeros, then the kept set (4 us; as a host-built row it was a 1 MB copy and three waits).
+__global__ void __launch_bounds__(256) dense_zero_kernel(float *out, int vocab) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < vocab) out[i] = 0.0f;
+}
+__global__ void __launch_bounds__(256) dense_scatter_kernel(float *out, int vocab, const uint32_t *res, const uint32_t *idx,
+                                                            const float *probs) {
+    const int n = min((int)res[0], vocab);
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) out[idx[i]] = probs[i];
 }
 
 __global__ void __launch_bounds__(256) make_keys_kernel(const float *lg, int vocab, uint64_t *out) {
@@ -133,8 +232,16 @@ __device__ float seq_sum(const float *p, int n, bool desc) {
     return s;
 }
 
+// Where the kept set's ids and probabilities are while one kernel works on them: the LDS for sets of up to LDS_SET
+// candidates (lane 0's ordered sums read them one by one), else the sampler's arrays.
+constexpr int LDS_SET = 512;
+struct KeptSet {
+    uint32_t *idx;
+    float *probs;
+};
+
 // sample.rs:181-236 `process` (not greedy): the kept set into idx/probs; returns its size. Whole work-group.
-__device__ int process(const SampArgs &a, const float *lg, const uint64_t *keys) {
+__device__ int process(const SampArgs &a, const KeptSet &ks, const float *lg, const uint64_t *keys) {
     __shared__ float s_sum;
     __shared__ int s_n, s_first;
     const int tid = threadIdx.x, nc = a.n_cand;
@@ -142,14 +249,14 @@ __device__ int process(const SampArgs &a, const float *lg, const uint64_t *keys)
     const float m = lg[(uint32_t)keys[0]] * inv_t;
     for (int i = tid; i < nc; i += ST) {
         const uint32_t id = (uint32_t)keys[i];
-        a.idx[i] = id;
-        a.probs[i] = aq_expf(lg[id] * inv_t - m);
+        ks.idx[i] = id;
+        ks.probs[i] = aq_expf(lg[id] * inv_t - m);
     }
     __syncthreads();
-    if (tid == 0) s_sum = seq_sum(a.probs, nc, true);
+    if (tid == 0) s_sum = seq_sum(ks.probs, nc, true);
     __syncthreads();
     const float sum = s_sum;
-    for (int i = tid; i < nc; i += ST) a.probs[i] = a.probs[i] / sum;
+    for (int i = tid; i < nc; i += ST) ks.probs[i] = ks.probs[i] / sum;
     __syncthreads();
     if (tid == 0) {
         int n = nc;
@@ -157,7 +264,7 @@ __device__ int process(const SampArgs &a, const float *lg, const uint64_t *keys)
             float cum = 0.0f;
             n = 0;
             while (n < nc && cum < a.cfg.top_p) {
-                cum += a.probs[n];
+                cum += ks.probs[n];
                 n++;
             }
             if (n < 1) n = 1;
@@ -168,48 +275,48 @@ __device__ int process(const SampArgs &a, const float *lg, const uint64_t *keys)
     __syncthreads();
     int n = s_n;
     if (a.cfg.min_p > 0.0f) { // the first candidate after the top one below min_p * p[0] ends the set
-        const float thr = a.cfg.min_p * a.probs[0];
+        const float thr = a.cfg.min_p * ks.probs[0];
         for (int i = 1 + tid; i < n; i += ST)
-            if (!(a.probs[i] >= thr)) atomicMin(&s_first, i);
+            if (!(ks.probs[i] >= thr)) atomicMin(&s_first, i);
         __syncthreads();
         n = s_first;
     }
-    if (tid == 0) s_sum = seq_sum(a.probs, n, true);
+    if (tid == 0) s_sum = seq_sum(ks.probs, n, true);
     __syncthreads();
     const float s = s_sum;
-    for (int i = tid; i < n; i += ST) a.probs[i] = a.probs[i] / s;
+    for (int i = tid; i < n; i += ST) ks.probs[i] = ks.probs[i] / s;
     __syncthreads();
     return n;
 }
 
 // sample.rs:239-251 `draw` (lane 0). `desc`: probs non-increasing (a processed set), so the running mass may stop
 // early: once it cannot grow, a u at or above it ends on the last kept id, as the reference's fall-through does.
-__device__ uint32_t draw(const SampArgs &a, int n, uint64_t rs[4], bool desc) {
+__device__ uint32_t draw(const KeptSet &ks, int n, uint64_t rs[4], bool desc) {
     const float u = rng_f32(rs);
     float cum = 0.0f;
     for (int i = 0; i < n; i++) {
-        const float p = a.probs[i];
+        const float p = ks.probs[i];
         if (desc && p < quarter_ulp(cum)) break;
         cum += p;
-        if (u < cum) return a.idx[i];
+        if (u < cum) return ks.idx[i];
     }
-    return a.idx[n - 1];
+    return ks.idx[n - 1];
 }
 
 // sample.rs:272-303 `accept_or_resample` after `process` left n kept: whole work-group; lane 0 returns the token.
-__device__ uint32_t accept(const SampArgs &a, const float *lg, const uint64_t *keys, const float *q, uint32_t d, int n,
-                           uint64_t rs[4], bool *ok_out) {
+__device__ uint32_t accept(const SampArgs &a, const KeptSet &ks, const float *lg, const uint64_t *keys,
+                           const float *q, uint32_t d, int n, uint64_t rs[4], bool *ok_out) {
     __shared__ int s_pos, s_ok;
     __shared__ float s_sum;
     const int tid = threadIdx.x;
     if (tid == 0) s_pos = -1;
     __syncthreads();
     for (int i = tid; i < n; i += ST)
-        if (a.idx[i] == d) s_pos = i;
+        if (ks.idx[i] == d) s_pos = i;
     __syncthreads();
     uint32_t tok = d;
     if (tid == 0) {
-        const float pd = s_pos >= 0 ? a.probs[s_pos] : 0.0f;
+        const float pd = s_pos >= 0 ? ks.probs[s_pos] : 0.0f;
         const float qd = q[d];
         const float u = rng_f32(rs);
         s_ok = (qd > 0.0f && (pd >= qd || u < pd / qd)) ? 1 : 0;
@@ -219,19 +326,19 @@ __device__ uint32_t accept(const SampArgs &a, const float *lg, const uint64_t *k
     *ok_out = ok;
     if (ok) return tok;
     // the residual max(0, p - q) over the kept set, renormalised
-    for (int i = tid; i < n; i += ST) a.probs[i] = fmaxf(a.probs[i] - q[a.idx[i]], 0.0f);
+    for (int i = tid; i < n; i += ST) ks.probs[i] = fmaxf(ks.probs[i] - q[ks.idx[i]], 0.0f);
     __syncthreads();
-    if (tid == 0) s_sum = seq_sum(a.probs, n, false);
+    if (tid == 0) s_sum = seq_sum(ks.probs, n, false);
     __syncthreads();
     const float sum = s_sum;
     if (!(sum > 0.0f)) { // p under q everywhere: the target's own distribution (sample.rs:293-297)
-        const int n2 = process(a, lg, keys);
-        if (tid == 0) tok = draw(a, n2, rs, true);
+        const int n2 = process(a, ks, lg, keys);
+        if (tid == 0) tok = draw(ks, n2, rs, true);
         return tok;
     }
-    for (int i = tid; i < n; i += ST) a.probs[i] = a.probs[i] / sum;
+    for (int i = tid; i < n; i += ST) ks.probs[i] = ks.probs[i] / sum;
     __syncthreads();
-    if (tid == 0) tok = draw(a, n, rs, false);
+    if (tid == 0) tok = draw(ks, n, rs, false);
     return tok;
 }
 
@@ -242,6 +349,18 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
         for (int i = 0; i < 4; i++) rs[i] = a.rng[i];
     __shared__ uint32_t s_tok;
     __shared__ int s_brk;
+    __shared__ float l_probs[LDS_SET];
+    __shared__ uint32_t l_idx[LDS_SET];
+    const bool lds = a.n_cand <= LDS_SET && a.op != OP_GREEDY_SET;
+    const KeptSet ks = lds ? KeptSet{l_idx, l_probs} : KeptSet{a.idx, a.probs};
+    auto keep = [&]() { // back to the sampler's arrays, for later calls
+        if (!lds) return;
+        __syncthreads();
+        for (int i = tid; i < a.n_cand; i += ST) {
+            a.idx[i] = l_idx[i];
+            a.probs[i] = l_probs[i];
+        }
+    };
     switch (a.op) {
     case OP_GREEDY_SET: // the greedy kept set: the argmax (already in res[1]) with probability 1
         if (tid == 0) {
@@ -254,7 +373,8 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
     case OP_PROCESS:
     case OP_SAMPLE:
     case OP_DRAFT: {
-        const int n = process(a, a.logits, a.keys);
+        const int n = process(a, ks, a.logits, a.keys);
+        keep();
         if (a.op == OP_PROCESS) {
             if (tid == 0) {
                 a.res[0] = (uint32_t)n;
@@ -263,7 +383,7 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
             return;
         }
         if (tid == 0) {
-            s_tok = draw(a, n, rs, true);
+            s_tok = draw(ks, n, rs, true);
             a.res[0] = (uint32_t)n;
             a.res[1] = s_tok;
             a.res[3] = 1;
@@ -274,8 +394,8 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
             for (uint32_t j = tid; j < old; j += ST) a.q_out[a.q_idx[j]] = 0.0f;
             __syncthreads();
             for (int j = tid; j < n; j += ST) {
-                a.q_out[a.idx[j]] = a.probs[j];
-                a.q_idx[j] = a.idx[j];
+                a.q_out[ks.idx[j]] = ks.probs[j];
+                a.q_idx[j] = ks.idx[j];
             }
             if (tid == 0) *a.q_n = (uint32_t)n;
         }
@@ -283,15 +403,16 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
     }
     case OP_DRAW:
         if (tid == 0) {
-            s_tok = draw(a, (int)a.res[0], rs, a.res[3] != 0);
+            s_tok = draw(KeptSet{a.idx, a.probs}, (int)a.res[0], rs, a.res[3] != 0);
             a.res[1] = s_tok;
             if (a.tok_out) *a.tok_out = s_tok;
         }
         break;
     case OP_ACCEPT: {
-        const int n = process(a, a.logits, a.keys);
+        const int n = process(a, ks, a.logits, a.keys);
         bool ok = false;
-        const uint32_t tok = accept(a, a.logits, a.keys, a.q, a.d, n, rs, &ok);
+        const uint32_t tok = accept(a, ks, a.logits, a.keys, a.q, a.d, n, rs, &ok);
+        keep();
         if (tid == 0) {
             a.res[0] = (uint32_t)n;
             a.res[1] = tok;
@@ -307,9 +428,9 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
         while (m < a.k) {
             const float *lg = a.logits + (size_t)m * v;
             const uint64_t *keys = a.keys + (size_t)m * a.key_stride;
-            const int n = process(a, lg, keys);
+            const int n = process(a, ks, lg, keys);
             bool ok = false;
-            const uint32_t tok = accept(a, lg, keys, a.q + (size_t)m * v, a.drafts[m], n, rs, &ok);
+            const uint32_t tok = accept(a, ks, lg, keys, a.q + (size_t)m * v, a.drafts[m], n, rs, &ok);
             if (tid == 0) {
                 a.emitted[m] = tok;
                 s_brk = ok ? 0 : 1;
@@ -319,9 +440,10 @@ __global__ void __launch_bounds__(ST) sampler_kernel(SampArgs a) {
             m++;
         }
         if (m == a.k) {
-            const int n = process(a, a.logits + (size_t)m * v, a.keys + (size_t)m * a.key_stride);
-            if (tid == 0) a.emitted[m] = draw(a, n, rs, true);
+            const int n = process(a, ks, a.logits + (size_t)m * v, a.keys + (size_t)m * a.key_stride);
+            if (tid == 0) a.emitted[m] = draw(ks, n, rs, true);
         }
+        keep();
         if (tid == 0) {
             a.info[0] = (uint32_t)m;
             a.info[1] = (uint32_t)(m + 1);
@@ -378,12 +500,13 @@ int candidates(aq_sampler *sp, const float *logits, int rows, hipStream_t st, co
     const int vocab = (int)sp->vocab, nc = n_cand_of(sp);
     if (nc <= KMAX_FAST) {
         int L = (vocab + SZ - 1) / SZ;
-        hipLaunchKernelGGL(topk_chunk_kernel, dim3(L, rows), dim3(ST), 0, st, logits, (size_t)vocab, vocab,
+        const auto select = nc <= KMAX_FEW ? topk_few_kernel : topk_chunk_kernel;
+        hipLaunchKernelGGL(select, dim3(L, rows), dim3(ST), 0, st, logits, (size_t)vocab, vocab,
                            (const uint64_t *)nullptr, (size_t)0, 0, nc, sp->bufa, sp->chunk_stride);
         uint64_t *in = sp->bufa, *out = sp->bufb;
         while (L > 1) { // every chunk of SZ keys keeps its first nc: the global first nc survive in their chunks
             const int L2 = (L * nc + SZ - 1) / SZ;
-            hipLaunchKernelGGL(topk_chunk_kernel, dim3(L2, rows), dim3(ST), 0, st, (const float *)nullptr, (size_t)0,
+            hipLaunchKernelGGL(select, dim3(L2, rows), dim3(ST), 0, st, (const float *)nullptr, (size_t)0,
                                vocab, (const uint64_t *)in, sp->chunk_stride, L * nc, nc, out, sp->chunk_stride);
             std::swap(in, out);
             L = L2;
@@ -680,19 +803,15 @@ int aq_sampler_sample(aq_sampler *sp, const float *logits_dev, uint32_t *tok) {
 int aq_sampler_write_dense(aq_sampler *sp, float *dense_dev) {
     AQ_REQUIRE(sp && dense_dev, "aq_sampler_write_dense: null argument");
     AQ_HIP(hipSetDevice(sp->device));
-    int rc = join(sp, sp->ctx->stream);
-    if (!rc) rc = sync_res(sp, sp->ctx->stream);
+    hipStream_t st = sp->ctx->stream;
+    const int rc = join(sp, st);
     if (rc) return rc;
-    // sample.rs:259-265: zeros, then the kept set (the operator-level form; the model writes it on the device)
-    const size_t nk = sp->pinned[0];
-    std::vector<uint32_t> ids(nk);
-    std::vector<float> pr(nk), dense((size_t)sp->vocab, 0.0f);
-    if (nk) {
-        AQ_HIP(hipMemcpy(ids.data(), sp->idx, nk * 4, hipMemcpyDeviceToHost));
-        AQ_HIP(hipMemcpy(pr.data(), sp->probs, nk * 4, hipMemcpyDeviceToHost));
-    }
-    for (size_t i = 0; i < nk; i++) dense[ids[i]] = pr[i];
-    AQ_HIP(hipMemcpy(dense_dev, dense.data(), dense.size() * 4, hipMemcpyHostToDevice));
+    const int vocab = (int)sp->vocab;
+    hipLaunchKernelGGL(dense_zero_kernel, dim3((vocab + 255) / 256), dim3(256), 0, st, dense_dev, vocab);
+    hipLaunchKernelGGL(dense_scatter_kernel, dim3(std::min((vocab + 255) / 256, 64)), dim3(256), 0, st, dense_dev, vocab,
+                       sp->res, sp->idx, sp->probs);
+    if (hipGetLastError() != hipSuccess) return fail(AQ_EHIP, "aq_sampler_write_dense: launch");
+    AQ_HIP(hipStreamSynchronize(st));
     return 0;
 }
 
