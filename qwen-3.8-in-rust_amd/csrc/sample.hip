@@ -166,7 +166,7 @@ __global__ void __launch_bounds__(ST) topk_few_kernel(const float *lg, size_t lg
     }
 }
 
-// `write_dense` (sample.rs:259-265): zeros, then the kept set (4 us; as a host-built row it was a 1 MB copy and three waits).
+// `write_dense` (sample.rs:259-265): zeros, then the kept set (4 us; a host-built row took a 1 MB copy and three waits).
 __global__ void __launch_bounds__(256) dense_zero_kernel(float *out, int vocab) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < vocab) out[i] = 0.0f;
