@@ -142,8 +142,12 @@ __device__ __forceinline__ float from_lane7(float v) {
 
 // Work-group (head, 32 columns): wave w columns 8 w .. 8 w + 7, lane = column * 8 + key part. deltanet.rs:43-86 per row:
 // S *= decay; kv = sum_k S k; delta = (v - kv) beta; S += k delta; o = sum_k S q. The next row's inputs are loaded while
-// this one's sums run.
-template <int DK>
+// this one's sums run. RAW: the isolated recurrence of a verify batch, inputs as given (4-byte aligned) and the state
+// written as it stands after row a.keep - 1 (keep 0: not at all) - one launch over 192 work-groups at 48 heads x 128 x 128,
+// where the heads' own work-groups ran every row and then the kept ones again: 10.5 us for 4 rows instead of 17.
+typedef float dn_f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int DK, bool RAW>
 __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
     constexpr int KH = DK / 8;
     const DnPre p = dn_pre(a);
@@ -156,20 +160,18 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
 #pragma unroll
     for (int u = 0; u < KH; u++) s[u] = srec[(size_t)u * dv];
     auto load = [&](int b, int i) {
-        const float *row = p.qkv + (size_t)i * p.cd;
-        const float *qs = row + kh * DK + j * KH, *ks = row + p.kd + kh * DK + j * KH;
+        const size_t at = (size_t)kh * DK + j * KH, e = (size_t)i * a.nv + h;
+        const float *qs = RAW ? a.rq + (size_t)i * p.kd + at : p.qkv + (size_t)i * p.cd + at;
+        const float *ks = RAW ? a.rk + (size_t)i * p.kd + at : p.qkv + (size_t)i * p.cd + p.kd + at;
         if constexpr (KH % 4 == 0) {
 #pragma unroll
             for (int u = 0; u < KH; u += 4) {
-                const float4 q4 = *reinterpret_cast<const float4 *>(qs + u), k4 = *reinterpret_cast<const float4 *>(ks + u);
-                q[b][u] = q4.x;
-                q[b][u + 1] = q4.y;
-                q[b][u + 2] = q4.z;
-                q[b][u + 3] = q4.w;
-                k[b][u] = k4.x;
-                k[b][u + 1] = k4.y;
-                k[b][u + 2] = k4.z;
-                k[b][u + 3] = k4.w;
+                const dn_f4u q4 = *reinterpret_cast<const dn_f4u *>(qs + u), k4 = *reinterpret_cast<const dn_f4u *>(ks + u);
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    q[b][u + w] = q4[w];
+                    k[b][u + w] = k4[w];
+                }
             }
         } else {
 #pragma unroll
@@ -178,9 +180,19 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
                 k[b][u] = ks[u];
             }
         }
-        v[b] = row[2 * p.kd + h * dv + c];
-        de[b] = p.decay[(size_t)i * a.nv + h];
-        be[b] = p.beta[(size_t)i * a.nv + h];
+        if constexpr (RAW) {
+            v[b] = a.rv[(size_t)i * p.vd + h * dv + c];
+            de[b] = exp_f(a.rg[e]);
+            be[b] = a.rbeta[e];
+        } else {
+            v[b] = p.qkv[(size_t)i * p.cd + 2 * p.kd + h * dv + c];
+            de[b] = p.decay[e];
+            be[b] = p.beta[e];
+        }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int u = 0; u < KH; u++) srec[(size_t)u * dv] = s[u];
     };
     auto step = [&](int b, int i) {
         float x[KH];
@@ -198,6 +210,7 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
         }
         const float o = lane_chain<KH>(x);
         if (j == 7) a.out[(size_t)i * p.vd + h * dv + c] = o;
+        if (RAW && i + 1 == a.keep) store();
     };
     load(0, 0);
     int i = 0;
@@ -208,8 +221,20 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
         step(1, i + 1);
     }
     if (i < a.t) step(0, i);
-#pragma unroll
-    for (int u = 0; u < KH; u++) srec[(size_t)u * dv] = s[u];
+    if (!RAW) store();
+}
+
+template <bool RAW>
+bool launch_recurrence(const DnArgs &a, hipStream_t stream) {
+    const dim3 grid((unsigned)(a.nv * ((a.dv + 31) / 32)));
+    switch (a.dk) {
+    case 8: hipLaunchKernelGGL((dn_recurrence_kernel<8, RAW>), grid, dim3(256), 0, stream, a); return true;
+    case 16: hipLaunchKernelGGL((dn_recurrence_kernel<16, RAW>), grid, dim3(256), 0, stream, a); return true;
+    case 32: hipLaunchKernelGGL((dn_recurrence_kernel<32, RAW>), grid, dim3(256), 0, stream, a); return true;
+    case 64: hipLaunchKernelGGL((dn_recurrence_kernel<64, RAW>), grid, dim3(256), 0, stream, a); return true;
+    case 128: hipLaunchKernelGGL((dn_recurrence_kernel<128, RAW>), grid, dim3(256), 0, stream, a); return true;
+    }
+    return false;
 }
 
 // Work-group (head, row): y = (w * (o * inv_rms(o))) * silu(z) (rmsnorm.rs:37-46) in place over the recurrence's output,
@@ -253,8 +278,8 @@ size_t dn_chunk_floats(const DnArgs &a) {
 }
 
 int launch_dn_chunk(const DnArgs &a, hipStream_t stream) {
-    AQ_REQUIRE(!a.raw && a.out && a.z && a.ssm_norm && a.pre && a.write_state && a.t >= 3 && a.t <= 4096,
-               "deltanet: more than 8 rows are a prompt chunk (projected gates, output, state written)");
+    AQ_REQUIRE(a.out && a.z && a.ssm_norm && a.pre && a.write_state && a.t >= 3 && a.t <= 4096,
+               "deltanet: more than 8 rows are a prompt chunk (output, state written)");
     AQ_REQUIRE(a.dv % 8 == 0 && a.dv <= 256 && 2 * a.dk <= 512 && ((uintptr_t)a.pre & 15) == 0 &&
                    ((uintptr_t)a.conv_w & 15) == 0,
                "deltanet: chunk shape");
@@ -262,18 +287,22 @@ int launch_dn_chunk(const DnArgs &a, hipStream_t stream) {
     hipLaunchKernelGGL(dn_inputs_kernel, dim3((unsigned)(a.nk + (vd + 255) / 256 + 1), (unsigned)a.t), dim3(256), 0, stream, a);
     int rc = launched("deltanet inputs");
     if (rc) return rc;
-    const dim3 grid((unsigned)(a.nv * ((a.dv + 31) / 32)));
-    switch (a.dk) {
-    case 8: hipLaunchKernelGGL(dn_recurrence_kernel<8>, grid, dim3(256), 0, stream, a); break;
-    case 16: hipLaunchKernelGGL(dn_recurrence_kernel<16>, grid, dim3(256), 0, stream, a); break;
-    case 32: hipLaunchKernelGGL(dn_recurrence_kernel<32>, grid, dim3(256), 0, stream, a); break;
-    case 64: hipLaunchKernelGGL(dn_recurrence_kernel<64>, grid, dim3(256), 0, stream, a); break;
-    case 128: hipLaunchKernelGGL(dn_recurrence_kernel<128>, grid, dim3(256), 0, stream, a); break;
-    default: return fail(AQ_EUNSUP, "deltanet: head dims (k, v) not built: " + std::to_string(a.dk) + ", " + std::to_string(a.dv));
-    }
+    if (!launch_recurrence<false>(a, stream))
+        return fail(AQ_EUNSUP, "deltanet: head dims (k, v) not built: " + std::to_string(a.dk) + ", " + std::to_string(a.dv));
     if ((rc = launched("deltanet recurrence"))) return rc;
     hipLaunchKernelGGL(dn_output_kernel, dim3((unsigned)a.nv, (unsigned)a.t), dim3(256), 0, stream, a);
     return launched("deltanet output");
+}
+
+int launch_dn_raw(const DnArgs &a, hipStream_t stream) {
+    AQ_REQUIRE(a.t >= 1 && a.nk >= 1 && a.nv >= 1 && a.nv % a.nk == 0, "deltanet: head counts");
+    AQ_REQUIRE(a.dv >= 1 && a.dv <= 256, "deltanet: head_dim_v must be 1..256");
+    AQ_REQUIRE(a.rec, "deltanet: no state");
+    AQ_REQUIRE(a.rq && a.rk && a.rv && a.rg && a.rbeta && a.out && a.keep <= a.t, "deltanet: raw inputs");
+    const bool built = a.dk == a.dv ? a.dk <= 128 : (a.dk == 128 && a.dv == 256) || (a.dk == 64 && a.dv == 128);
+    if (!built || !launch_recurrence<true>(a, stream))
+        return fail(AQ_EUNSUP, "deltanet: head dims (k, v) not built: " + std::to_string(a.dk) + ", " + std::to_string(a.dv));
+    return launched("deltanet recurrence");
 }
 
 } // namespace aq

@@ -1634,7 +1634,6 @@ int aq_deltanet_verify_commit_dev(aq_ctx *ctx, uint32_t nk, uint32_t nv, uint32_
     AQ_REQUIRE(nk >= 1 && nv % nk == 0, "aq_deltanet_verify_commit: heads");
     AQ_HIP(hipSetDevice(ctx->device));
     DnArgs d;
-    d.raw = 1;
     d.rq = q_dev;
     d.rk = k_dev;
     d.rv = v_dev;
@@ -1645,18 +1644,11 @@ int aq_deltanet_verify_commit_dev(aq_ctx *ctx, uint32_t nk, uint32_t nv, uint32_
     d.nv = (int)nv;
     d.dk = (int)dk;
     d.dv = (int)dv;
-    // verify: every row's output from the committed state, the state untouched
+    // every row's output from the committed state; the state left as it stands after the kept rows
     d.t = (int)t;
-    d.write_state = 0;
+    d.keep = (int)keep;
     d.out = out_dev;
-    int rc = launch_dn_core(d, ctx->stream);
-    // commit: the kept rows again, state written (the outputs of the kept rows are recomputed identically)
-    if (!rc && keep > 0) {
-        d.t = (int)keep;
-        d.write_state = 1;
-        d.out = nullptr;
-        rc = launch_dn_core(d, ctx->stream);
-    }
+    int rc = launch_dn_raw(d, ctx->stream);
     if (hipStreamSynchronize(ctx->stream) != hipSuccess && !rc) rc = fail(AQ_EHIP, "deltanet: sync");
     return rc;
 }

@@ -72,19 +72,21 @@ struct DnArgs {
     int out_q80 = 0;      // also the Q8_0 form of `out` into q80 (its rows = the t rows; vd and dv multiples of 32)
     Act q80;
     int t = 0, nk = 0, nv = 0, dk = 0, dv = 0, kernel = 0;
-    // raw mode (the isolated recurrence): q, k (t x nk*dk), v (t x nv*dv), g, beta (t x nv) used as given
-    int raw = 0;
+    // the isolated recurrence: q, k (t x nk*dk), v (t x nv*dv), g, beta (t x nv) used as given; the state is written as
+    // it stands after `keep` rows (0: not written)
+    int keep = 0;
     const float *rq = nullptr, *rk = nullptr, *rv = nullptr, *rg = nullptr, *rbeta = nullptr;
     const uint32_t *t_dev = nullptr; // multi launch: the row count, read on the device (1..8)
     float *pre = nullptr; // prompt chunks: dn_chunk_floats of scratch
 };
 // t rows, up to 8 in one launch; more (a prompt chunk) by launch_dn_chunk.
 int launch_dn_core(const DnArgs &a, hipStream_t stream);
-// A prompt chunk's rows (deltanet_chunk.hip): projected gates (no raw mode), `pre` set, the state and the conv window
-// written.
+// A prompt chunk's rows (deltanet_chunk.hip): `pre` set, the state and the conv window written.
 int launch_dn_chunk(const DnArgs &a, hipStream_t stream);
 // Floats of `pre` for t rows.
 size_t dn_chunk_floats(const DnArgs &a);
+// The isolated recurrence over t rows (r* inputs, `out`, `keep`), one launch (deltanet_chunk.hip).
+int launch_dn_raw(const DnArgs &a, hipStream_t stream);
 // n DnArgs (device array, commit form: saved gates, no output), all with the head shape of `like`: one launch.
 int launch_dn_core_multi(const DnArgs *args_dev, const DnArgs &like, int n, hipStream_t stream);
 

@@ -426,23 +426,21 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
     static_assert(TT >= 0 && TT <= DN_TMAX, "rows per launch");
     constexpr int TM = TT ? TT : DN_TMAX; // the input loops' bound
     const int t = TT ? TT : t_in;
-    const bool raw_ = a.raw;
     static_assert(DK <= 256 && DV <= 256 && DN_THREADS >= 448 && DN_TMAX * 2 <= 16, "DeltaNet work-group shape");
     __shared__ float sq[DN_TMAX][DK], sk[DN_TMAX][DK], sv[DN_TMAX][DV], sz[DN_TMAX][DV], so[DN_TMAX][DV];
     __shared__ float rdec[DN_TMAX], rbeta[DN_TMAX], rq[DN_TMAX], rk[DN_TMAX], ro[DN_TMAX];
     const int j = threadIdx.x, lane = j & 63, wave = j >> 6;
     const int kh = p % a.nk;
     const int kd = a.nk * DK, vd = a.nv * DV, cd = 2 * kd + vd;
-    const bool gated = a.out && !raw_;
+    const bool gated = a.out;
     // the gate inputs, loaded before phase A so their latency hides behind it: wave 5 computes the decays and
     // wave 7 the betas (lane i = row i), each in its own wave so neither waits for the other's branch
     const bool gate_lane = (wave == 5 || wave == 7) && lane < t;
     const int gr = wave == 5 ? 0 : 1;
     float gv = 0.0f, gsa = 0.0f, gdt = 0.0f;
     if (gate_lane) {
-        gv = raw_ ? (gr == 0 ? a.rg : a.rbeta)[(size_t)lane * a.nv + p]
-                  : (gr == 0 ? a.a : a.b)[(size_t)lane * a.nv + p];
-        if (gr == 0 && !raw_) {
+        gv = (gr == 0 ? a.a : a.b)[(size_t)lane * a.nv + p];
+        if (gr == 0) {
             gsa = a.ssm_a[p];
             gdt = a.dt_bias[p];
         }
@@ -461,62 +459,50 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
     }
 
     // ---- A: channels over all rows
-    if (raw_) {
-        for (int e = j; e < t * DK; e += DN_THREADS) {
-            const int i = e / DK, c = e % DK;
-            sq[i][c] = a.rq[(size_t)i * kd + kh * DK + c];
-            sk[i][c] = a.rk[(size_t)i * kd + kh * DK + c];
-        }
-        for (int e = j; e < t * DV; e += DN_THREADS) {
-            const int i = e / DV, c = e % DV;
-            sv[i][c] = a.rv[(size_t)i * vd + p * DV + c];
-        }
-    } else {
-        // task c: q channel c (c < DK), k channel c - DK, v channel c - 2 DK (conv, conv.rs:11-36), then the
-        // z channels (silu only)
-        const int n_conv = 2 * DK + DV, n_task = n_conv + (gated ? DV : 0);
-        for (int c = j; c < n_task; c += DN_THREADS) {
-            if (c < n_conv) {
-                const int kind = c < DK ? 0 : c < 2 * DK ? 1 : 2;
-                const int cc = kind == 2 ? c - 2 * DK : c - kind * DK;
-                const int ch = kind == 0 ? kh * DK + cc : kind == 1 ? kd + kh * DK + cc : 2 * kd + p * DV + cc;
-                float seq[TM + 3];
+    // task c: q channel c (c < DK), k channel c - DK, v channel c - 2 DK (conv, conv.rs:11-36), then the
+    // z channels (silu only)
+    const int n_conv = 2 * DK + DV, n_task = n_conv + (gated ? DV : 0);
+    for (int c = j; c < n_task; c += DN_THREADS) {
+        if (c < n_conv) {
+            const int kind = c < DK ? 0 : c < 2 * DK ? 1 : 2;
+            const int cc = kind == 2 ? c - 2 * DK : c - kind * DK;
+            const int ch = kind == 0 ? kh * DK + cc : kind == 1 ? kd + kh * DK + cc : 2 * kd + p * DV + cc;
+            float seq[TM + 3];
 #pragma unroll
-                for (int e = 0; e < 3; e++)
-                    seq[e] = a.conv_src[(size_t)ch * 3 + e];
-                float cw[4];
+            for (int e = 0; e < 3; e++)
+                seq[e] = a.conv_src[(size_t)ch * 3 + e];
+            float cw[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) cw[e] = a.conv_w[(size_t)ch * 4 + e];
+            for (int e = 0; e < 4; e++) cw[e] = a.conv_w[(size_t)ch * 4 + e];
 #pragma unroll
-                for (int i = 0; i < TM; i++) seq[3 + i] = a.mixed[(size_t)(i < t ? i : t - 1) * cd + ch];
-                float *dst = kind == 0 ? &sq[0][cc] : kind == 1 ? &sk[0][cc] : &sv[0][cc];
-                const int dstride = kind == 2 ? DV : DK;
+            for (int i = 0; i < TM; i++) seq[3 + i] = a.mixed[(size_t)(i < t ? i : t - 1) * cd + ch];
+            float *dst = kind == 0 ? &sq[0][cc] : kind == 1 ? &sk[0][cc] : &sv[0][cc];
+            const int dstride = kind == 2 ? DV : DK;
 #pragma unroll
-                for (int i = 0; i < TM; i++) {
-                    if (i < t) {
-                        float acc = 0.0f;
-                        acc += cw[0] * seq[i];
-                        acc += cw[1] * seq[i + 1];
-                        acc += cw[2] * seq[i + 2];
-                        acc += cw[3] * seq[i + 3];
-                        dst[i * dstride] = silu_f(acc);
-                    }
+            for (int i = 0; i < TM; i++) {
+                if (i < t) {
+                    float acc = 0.0f;
+                    acc += cw[0] * seq[i];
+                    acc += cw[1] * seq[i + 1];
+                    acc += cw[2] * seq[i + 2];
+                    acc += cw[3] * seq[i + 3];
+                    dst[i * dstride] = silu_f(acc);
                 }
-                if (a.conv_dst && (kind == 2 || p == kh)) {
-#pragma unroll
-                    for (int i = 0; i <= TM; i++) // the window after row t - 1: seq[t .. t + 2]
-                        if (i == t)
-                            for (int e = 0; e < 3; e++) a.conv_dst[(size_t)ch * 3 + e] = seq[i + e];
-                }
-            } else {
-                const int cc = c - n_conv;
-                float zr[TM];
-#pragma unroll
-                for (int i = 0; i < TM; i++) zr[i] = a.z[(size_t)(i < t ? i : t - 1) * vd + p * DV + cc];
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-                    if (i < t) sz[i][cc] = silu_f(zr[i]);
             }
+            if (a.conv_dst && (kind == 2 || p == kh)) {
+#pragma unroll
+                for (int i = 0; i <= TM; i++) // the window after row t - 1: seq[t .. t + 2]
+                    if (i == t)
+                        for (int e = 0; e < 3; e++) a.conv_dst[(size_t)ch * 3 + e] = seq[i + e];
+            }
+        } else {
+            const int cc = c - n_conv;
+            float zr[TM];
+#pragma unroll
+            for (int i = 0; i < TM; i++) zr[i] = a.z[(size_t)(i < t ? i : t - 1) * vd + p * DV + cc];
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+                if (i < t) sz[i][cc] = silu_f(zr[i]);
         }
     }
     __syncthreads();
@@ -527,7 +513,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
         // 6 (8-15): lane m of the chain holds its terms m*T .. m*T + T - 1 as registers and the running sum moves
         // one lane up after each lane's terms (DPP row shift), so lane 7 of the group ends with the whole sum,
         // added in order
-        if ((wave == 4 || wave == 6) && !raw_) {
+        if (wave == 4 || wave == 6) {
             constexpr int T = DK / 8;
             const int c = (wave == 4 ? 0 : 8) + (lane >> 3), m = lane & 7, cc = c < 2 * t ? c : 0;
             const float4 *x4 = reinterpret_cast<const float4 *>((cc & 1) ? sk[cc >> 1] : sq[cc >> 1]) + m * (T / 4);
@@ -556,7 +542,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
                     rq[c >> 1] = inv;
             }
         }
-    } else if (wave == 4 && !raw_ && lane < 2 * t) { // one sum per lane
+    } else if (wave == 4 && lane < 2 * t) { // one sum per lane
         const int i = lane >> 1;
         const float ss = seq_sum<true>((lane & 1) ? sk[i] : sq[i], 0, DK, 1, 0.0f);
         const float inv = 1.0f / sqrtf(ss + 1e-6f); // deltanet.rs:19-29 l2norm
@@ -569,21 +555,19 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
         const int i = lane;
         const float v = gv;
         if (gr == 0) {
-            const float g = raw_ ? v : gsa * softplus_f(v + gdt); // deltanet.rs:32-35 gate_g
+            const float g = gsa * softplus_f(v + gdt); // deltanet.rs:32-35 gate_g
             rdec[i] = exp_f(g);
         } else {
-            rbeta[i] = raw_ ? v : sigmoid_f(v);
+            rbeta[i] = sigmoid_f(v);
         }
     }
     __syncthreads();
-    if (!raw_) {
-        for (int e = j; e < t * DK; e += DN_THREADS) {
-            const int i = e / DK, cc = e % DK;
-            sq[i][cc] = (sq[i][cc] * rq[i]) * a.qscale;
-            sk[i][cc] = sk[i][cc] * rk[i];
-        }
-        __syncthreads();
+    for (int e = j; e < t * DK; e += DN_THREADS) {
+        const int i = e / DK, cc = e % DK;
+        sq[i][cc] = (sq[i][cc] * rq[i]) * a.qscale;
+        sk[i][cc] = sk[i][cc] * rk[i];
     }
+    __syncthreads();
 
     // ---- C: the recurrence of column c (deltanet.rs:43-86), row after row. Each part updates its keys' state and
     // forms their products in parallel (S *= decay, S k; then S += k delta, S q); the two sums over k stay one
@@ -640,13 +624,7 @@ __device__ __forceinline__ void dn_core_body(const DnArgs &a, const int p, const
                 if (hh > 0) ov = xfer2[c];
 #pragma unroll
                 for (int k = 0; k < KH; k++) ov += pk[k];
-                if (hh + 1 < H) {
-                    xfer2[c] = ov;
-                } else if (raw_) {
-                    if (a.out) a.out[(size_t)i * vd + p * DV + c] = ov;
-                } else {
-                    so[i][c] = ov;
-                }
+                (hh + 1 < H ? xfer2[c] : so[i][c]) = ov;
             }
             if (hh + 1 < H) __syncthreads();
         }
@@ -1156,17 +1134,12 @@ int launch_dn_core(const DnArgs &a, hipStream_t stream) {
     AQ_REQUIRE(a.t >= 1 && a.nk >= 1 && a.nv >= 1 && a.nv % a.nk == 0, "deltanet: head counts");
     AQ_REQUIRE(a.dv >= 1 && a.dv <= 256, "deltanet: head_dim_v must be 1..256");
     AQ_REQUIRE(a.rec, "deltanet: no state");
-    if (!a.raw) {
-        AQ_REQUIRE(a.kernel == 4, "deltanet: conv kernel must be 4 in this build");
-        AQ_REQUIRE(a.mixed && a.a && a.b && a.conv_src && a.conv_w && a.ssm_a && a.dt_bias, "deltanet: inputs");
-        AQ_REQUIRE(!a.out || (a.z && a.ssm_norm), "deltanet: output needs z and ssm_norm");
-        AQ_REQUIRE(!a.out_q80 || (a.out && a.dv % 32 == 0 && a.q80.q0 && a.q80.n == (size_t)a.nv * a.dv &&
-                                  a.q80.ncols >= (size_t)a.t),
-                   "deltanet: Q8_0 output needs whole 32-blocks and a buffer of t rows of nv * dv");
-    } else {
-        AQ_REQUIRE(a.rq && a.rk && a.rv && a.rg && a.rbeta, "deltanet: raw inputs");
-    }
-    AQ_REQUIRE(a.raw || (a.a && a.b), "deltanet: gate inputs");
+    AQ_REQUIRE(a.kernel == 4, "deltanet: conv kernel must be 4 in this build");
+    AQ_REQUIRE(a.mixed && a.a && a.b && a.conv_src && a.conv_w && a.ssm_a && a.dt_bias, "deltanet: inputs");
+    AQ_REQUIRE(!a.out || (a.z && a.ssm_norm), "deltanet: output needs z and ssm_norm");
+    AQ_REQUIRE(!a.out_q80 || (a.out && a.dv % 32 == 0 && a.q80.q0 && a.q80.n == (size_t)a.nv * a.dv &&
+                              a.q80.ncols >= (size_t)a.t),
+               "deltanet: Q8_0 output needs whole 32-blocks and a buffer of t rows of nv * dv");
     const int threads = DN_THREADS;
     const int key = a.dk * 1000 + a.dv;
     switch (key) {
@@ -1191,7 +1164,7 @@ int launch_dn_core(const DnArgs &a, hipStream_t stream) {
 
 int launch_dn_core_multi(const DnArgs *args_dev, const DnArgs &like, int n, hipStream_t stream) {
     AQ_REQUIRE(n >= 1 && args_dev, "deltanet: no layers");
-    AQ_REQUIRE(!like.raw && !like.out, "deltanet multi: commit form only (saved gates, no output)");
+    AQ_REQUIRE(!like.out, "deltanet multi: commit form only (saved gates, no output)");
     const int key = like.dk * 1000 + like.dv;
     switch (key) {
 #define AQ_DN(K, V)                                                                                           \
