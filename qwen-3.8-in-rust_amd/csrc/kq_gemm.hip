@@ -16,8 +16,8 @@
 // too: d = dx * d and -dx * dmin of a 16 x 64 tile are one K = 1 f32 outer product each (rounded once, no FMA), and
 // the Q4_K / Q5_K min sums prod[i] one K = 4 product of the mins and the group sums.
 //
-// Q8_0 / Q4_0 x Q8_0 (dot.rs:29-66): one product over K = 32 is one block's exact i32 sum for the tile (Q4_0: the
-// unsigned codes, less 8 * the activation block's code sum), then acc += (dw * dx) * f32(isum) per output.
+// Q8_0 / Q4_0 x Q8_0 (dot.rs:29-66): one product over K = 32 is one block's exact i32 sum for the tile (Q4_0: of the
+// codes less 8), then acc += (dw * dx) * f32(isum) per output.
 //
 // Work (K-quants): a work-group of eight waves owns two 16-row tiles x CT 16-column tiles; wave (rt, w) takes the lane
 // slots w and w + 4 (and min lane w) of row tile rt, for all of K. The eight lane chains are independent until the final
@@ -62,8 +62,6 @@ struct GemmArgs {
     // Q8_K activations (lane-slot order) or Q8_0 (natural order)
     const int8_t *xq;
     const float *xd;
-    const int16_t *xbs, *xq8s;
-    const int32_t *xs0;
     size_t n;
     // the many-column Q8_K form (Act::gh, gm; gcap columns)
     const uint16_t *gh;
@@ -76,12 +74,11 @@ struct GemmArgs {
 
 // ---- LDS staging ----
 // Operands reach the LDS by direct global-to-LDS copies (global_load_lds_*: each active lane's 16 or 4 bytes land at
-// m0 + 16 * lane or m0 + 4 * lane), issued GEMM_STAGES - 1 steps ahead into a ring of GEMM_STAGES buffers, so the
+// m0 + 16 * lane or m0 + 4 * lane), issued a ring's buffers less one ahead, so the
 // loads' latency is covered without holding the data in registers. Every wave issues the same number of copies per
 // step (a whole wave never skips one), so its count of outstanding vector-memory operations says which step has
 // landed; a work-group barrier after the wait makes every wave's copies of that step visible and, at the same
 // time, frees the buffer read one step earlier for the next copies.
-constexpr int GEMM_STAGES = 3;
 constexpr int GEMM_CUS = 256;
 
 __device__ __forceinline__ void dma16(uint32_t lds, const void *g) {
@@ -451,112 +448,128 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
     else kq_gemm_body<T, 1>(a, gm_lds, 32 * (a.nfull + k / CT), k % CT);
 }
 
-// One step of a Q8_0 / Q4_0 work-group = 8 blocks (256 elements), in 16-byte units: codes unit q * 16 + i = byte
-// chunk q of row r0 + i's 8 blocks (Q8_0: 16 chunks, Q4_0: 8), then row i's 8 f16 d at unit NQ + i; per wave the
-// activation codes as for the K-quants, then each column's 8 f32 d (32 B) and, for Q4_0, its 8 i32 code sums.
+// One step of a Q8_0 / Q4_0 work-group (32 rows x 64 columns, 8 waves of one 16 x 16 tile each) = 8 blocks (256
+// elements). In the LDS a row's or column's codes of the step are one run (256 bytes; Q4_0 rows 128), its 16-byte chunk q
+// at position q ^ the row's or column's number in the tile (Q4_0: of its pair), so that a copy's lanes read whole runs
+// from memory and the tile's 16 lanes read 16 different bank groups. Then per wave a region of 20 units: the 8 f32 d of 8
+// of its tile's columns, and the 8 f16 d of 4 of the work-group's rows.
 template <int T>
 struct Q8Stage {
     static constexpr int QC = T == AQ_TYPE_Q8_0 ? 16 : 8; // code chunks per row
-    static constexpr int W_UNITS = 16 * QC + 16;
-    static constexpr int WL = W_UNITS / 4;          // weight units per wave
-    static constexpr int WI = (WL + 63) / 64;       // copies they take
-    static constexpr int WB = W_UNITS * 16;
-    static constexpr int XB = 4096 + 512 + (T == AQ_TYPE_Q4_0 ? 512 : 0);
-    static constexpr int BYTES = WB + 4 * XB;
-    static constexpr int NDMA = WI + 5 + (T == AQ_TYPE_Q4_0 ? 1 : 0);
+    static constexpr int WB = 32 * QC * 16, XB = 64 * 256, DB = 320;
+    static constexpr int BYTES = WB + XB + 8 * DB;
+    static constexpr int RING = 3; // stages; two work-groups' rings fit a CU (six, one work-group each: no faster)
 };
 
+// Four copies per wave, or two where its column tile is past the columns.
 template <int T>
-__device__ __forceinline__ void q8_issue(const GemmArgs &a, uint32_t buf, size_t st, int r0, int c0w, int wave,
-                                         int lane) {
+__device__ __forceinline__ void q8_issue(const GemmArgs &a, uint32_t buf, size_t st, int r0, int c0, int wave, int lane,
+                                         bool xlive) {
     using S = Q8Stage<T>;
     const size_t nb = (size_t)a.nb; // 32-blocks per row
-#pragma unroll
-    for (int i = 0; i < S::WI; i++) {
-        if (i * 64 + lane < S::WL) { // every copy has active lanes: WL > 64 (WI - 1)
-            const int u = wave * S::WL + i * 64 + lane;
-            const uint8_t *src;
-            if (u < 16 * S::QC) {
-                const size_t row = (size_t)min(r0 + (u & 15), a.rows - 1);
-                src = a.qa + (row * nb + st * 8) * (S::QC * 2) + (size_t)(u >> 4) * 16;
-            } else {
-                const size_t row = (size_t)min(r0 + u - 16 * S::QC, a.rows - 1);
-                src = a.dm + (row * nb + st * 8) * 2;
-            }
-            dma16(uni(buf + (uint32_t)((wave * S::WL + i * 64) * 16)), src);
-        }
+    if (T == AQ_TYPE_Q8_0 || lane < 32) { // four rows' codes
+        const int i = 4 * wave + lane / S::QC, p = lane % S::QC, q = p ^ (T == AQ_TYPE_Q8_0 ? i & 15 : (i >> 1) & 7);
+        const size_t row = (size_t)min(r0 + i, a.rows - 1);
+        dma16(uni(buf + (uint32_t)(wave * 64 * S::QC)), a.qa + (row * nb + st * 8) * (S::QC * 2) + (size_t)q * 16);
     }
-    const uint32_t xw = buf + (uint32_t)(S::WB + wave * S::XB);
-    const size_t col = (size_t)min(c0w + (lane & 15), a.ncols - 1);
-    const int8_t *xs = a.xq + col * a.n + st * 256;
 #pragma unroll
-    for (int i = 0; i < 4; i++) dma16(uni(xw + (uint32_t)(i * 1024)), xs + (size_t)(i * 4 + (lane >> 4)) * 16);
-    const size_t c2 = (size_t)min(c0w + (lane >> 1), a.ncols - 1);
-    if (lane < 32) dma16(uni(xw + 4096), a.xd + c2 * nb + st * 8 + 4 * (lane & 1));
-    if constexpr (T == AQ_TYPE_Q4_0) {
-        if (lane < 32) dma16(uni(xw + 4608), a.xs0 + c2 * nb + st * 8 + 4 * (lane & 1));
+    for (int u = 0; u < 2 && xlive; u++) { // eight columns' codes
+        const int i = 8 * wave + 4 * u + (lane >> 4);
+        const size_t col = (size_t)min(c0 + i, a.ncols - 1);
+        dma16(uni(buf + (uint32_t)(S::WB + (2 * wave + u) * 1024)),
+              a.xq + col * a.n + st * 256 + (size_t)(((lane & 15) ^ i) & 15) * 16);
+    }
+    if (lane < 20) {
+        const size_t col = (size_t)min(c0 + 8 * wave + (lane >> 1), a.ncols - 1);
+        const size_t row = (size_t)min(r0 + 4 * wave + (lane & 3), a.rows - 1);
+        const uint8_t *xs = reinterpret_cast<const uint8_t *>(a.xd + col * nb + st * 8 + 4 * (lane & 1));
+        dma16(uni(buf + (uint32_t)(S::WB + S::XB + wave * S::DB)), lane < 16 ? xs : a.dm + (row * nb + st * 8) * 2);
     }
 }
 
-// Q8_0 / Q4_0 weights x Q8_0 activations: the same work-group and lane roles; one product over K = 32 per block.
+// Q8_0 / Q4_0 weights x Q8_0 activations: one product over K = 32 per block (v_mfma_i32_16x16x32_i8), its factors
+// d * d of four blocks at once as outer products (v_mfma_f32_16x16x1 with a zero addend: each rounded once), so a thread
+// is left with its four outputs' conversion, product and add per block. Q4_0's codes less 8 (dot.rs:48-66) enter as the
+// signed bytes 16 (code - 8) - one shift and one and-xor of the packed byte - and the weights' d divided by 16, both exact.
+// As 16 rows and four waves per work-group, one work-group per CU, the columns passed through the LDS for every 16 rows
+// (~7.5 TB/s of cache reads) and the factors were 12 of 28 vector operations per block. 64 columns: Q4_0 17408 x 5120
+// 92 -> 51 us, 5120 x 17408 119 -> 67, 12288 x 5120 52 -> 33; Q8_0 5120 x 6144 37 -> 24. Bound by a wave's own latency per
+// step (two waves per SIMD at 5120 rows: 0.75 us of it without any copies, the copies alone 0.4).
 template <int T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) q8_gemm_kernel(GemmArgs a) {
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) q8_gemm_kernel(GemmArgs a) {
     using S = Q8Stage<T>;
     extern __shared__ __align__(16) uint8_t gm_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int g = lane >> 4, li = lane & 15;
-    const int r0 = (int)blockIdx.x * 16;
-    const int c0w = (int)blockIdx.y * 64 + wave * 16;
-    const bool live = c0w < a.ncols;
+    const int g = lane >> 4, li = lane & 15, ct = wave & 3, rt = wave >> 2;
+    const int r0 = (int)blockIdx.x * 32;
+    const int c0 = (int)blockIdx.y * 64;
+    const bool live = c0 + 16 * ct < a.ncols;
+    const bool xlive = c0 + 16 * (wave >> 1) < a.ncols; // the tile whose columns this wave copies
     const int nst = a.nb / 8; // steps
     const uint32_t lds0 = (uint32_t)(uintptr_t)gm_lds;
+    const int wrow = 16 * rt + li, wx = T == AQ_TYPE_Q8_0 ? li : li >> 1;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int s = 0; s < GEMM_STAGES - 1; s++)
-        if (s < nst) q8_issue<T>(a, lds0 + (uint32_t)(s * S::BYTES), (size_t)s, r0, c0w, wave, lane);
+    for (int s = 0; s < S::RING - 1; s++)
+        if (s < nst) q8_issue<T>(a, lds0 + (uint32_t)(s * S::BYTES), (size_t)s, r0, c0, wave, lane, xlive);
 
+    int slot = 0;
     for (int st = 0; st < nst; st++) {
-        if (st + GEMM_STAGES - 2 < nst) wait_vm_barrier<(GEMM_STAGES - 2) * S::NDMA>();
-        else wait_vm_barrier<0>();
-        if (st + GEMM_STAGES - 1 < nst)
-            q8_issue<T>(a, lds0 + (uint32_t)(((st + GEMM_STAGES - 1) % GEMM_STAGES) * S::BYTES),
-                        (size_t)(st + GEMM_STAGES - 1), r0, c0w, wave, lane);
+        if (st + S::RING - 2 >= nst) wait_vm_barrier<0>();
+        else if (xlive) wait_vm_barrier<(S::RING - 2) * 4>();
+        else wait_vm_barrier<(S::RING - 2) * 2>();
+        if (st + S::RING - 1 < nst)
+            q8_issue<T>(a, lds0 + (uint32_t)((slot == 0 ? S::RING - 1 : slot - 1) * S::BYTES), (size_t)(st + S::RING - 1),
+                        r0, c0, wave, lane, xlive);
+        const uint8_t *W = gm_lds + slot * S::BYTES;
+        slot = slot == S::RING - 1 ? 0 : slot + 1;
         if (!live) continue;
-        const uint8_t *W = gm_lds + (st % GEMM_STAGES) * S::BYTES;
-        const uint8_t *X = W + S::WB + wave * S::XB;
-        uint4 dwr[4];
+        const uint8_t *X = W + S::WB + ct * 4096 + li * 256, *D = W + S::WB + S::XB;
+        const uint8_t *dw = D + (wrow >> 2) * S::DB + 256 + (li & 3) * 16 + g * 2;
+        const uint8_t *dx = D + (2 * ct + (li >> 3)) * S::DB + (li & 7) * 32 + g * 4;
+        W += wrow * (16 * S::QC) + 8 * (g & 1);
+        X += 8 * (g & 1);
+        // operands, then products, then the chains: left to itself the compiler ties each block's chain to its own reads
+        uint64_t wv[8], xv[8];
+        float dv[2], dxv[2];
 #pragma unroll
-        for (int j = 0; j < 4; j++) dwr[j] = *reinterpret_cast<const uint4 *>(W + (16 * S::QC + 4 * g + j) * 16);
+        for (int h = 0; h < 2; h++) {
+            dv[h] = h2f(*reinterpret_cast<const uint16_t *>(dw + 8 * h));
+            dxv[h] = *reinterpret_cast<const float *>(dx + 16 * h);
+        }
 #pragma unroll
         for (int b = 0; b < 8; b++) {
-            uint64_t wa;
-            if constexpr (T == AQ_TYPE_Q8_0) {
-                wa = *reinterpret_cast<const uint64_t *>(W + ((2 * b + (g >> 1)) * 16 + li) * 16 + 8 * (g & 1));
-            } else {
-                // elements 8g .. 8g + 7: bytes 8 (g & 1) .., low nibbles for g < 2, high for g >= 2
-                const uint64_t w = *reinterpret_cast<const uint64_t *>(W + (b * 16 + li) * 16 + 8 * (g & 1));
-                wa = (w >> (4 * (g >> 1))) & 0x0F0F0F0F0F0F0F0Full;
-            }
-            const uint64_t bx =
-                *reinterpret_cast<const uint64_t *>(X + ((2 * b + (g >> 1)) * 16 + li) * 16 + 8 * (g & 1));
-            const float dx = *reinterpret_cast<const float *>(X + 4096 + 32 * li + 4 * b);
-            int off = 0;
-            if constexpr (T == AQ_TYPE_Q4_0) // dot.rs:48-66: codes less 8
-                off = 8 * *reinterpret_cast<const int32_t *>(X + 4608 + 32 * li + 4 * b);
-            v4i c = {0, 0, 0, 0};
-            c = mma(wa, bx, c);
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t dww = (b >> 1) == 0 ? dwr[j].x : (b >> 1) == 1 ? dwr[j].y : (b >> 1) == 2 ? dwr[j].z : dwr[j].w;
-                acc[j] += (h2f(dww >> (16 * (b & 1))) * dx) * (float)(c[j] - off);
-            }
+            if constexpr (T == AQ_TYPE_Q8_0) wv[b] = *reinterpret_cast<const uint64_t *>(W + ((2 * b + (g >> 1)) ^ wx) * 16);
+            else wv[b] = *reinterpret_cast<const uint64_t *>(W + (b ^ wx) * 16);
+            xv[b] = *reinterpret_cast<const uint64_t *>(X + ((2 * b + (g >> 1)) ^ li) * 16);
         }
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16 f[2];
+        v4i c[8];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            f[h] = __builtin_amdgcn_mfma_f32_16x16x1f32(T == AQ_TYPE_Q4_0 ? dv[h] * 0.0625f : dv[h], dxv[h], f32x16{}, 0, 0, 0);
+#pragma unroll
+        for (int b = 0; b < 8; b++) {
+            uint64_t wa = wv[b];
+            if constexpr (T == AQ_TYPE_Q4_0) { // elements 8g .. 8g + 7: bytes 8 (g & 1) .., low nibbles for g < 2, else high
+                const int sh = g < 2 ? 4 : 0;
+                wa = pack2((((uint32_t)wa << sh) & 0xF0F0F0F0u) ^ 0x80808080u,
+                           (((uint32_t)(wa >> 32) << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
+            }
+            c[b] = mma(wa, xv[b], v4i{0, 0, 0, 0});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < 8; b++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[j] += f[b >> 2][4 * (b & 3) + j] * (float)c[b][j];
     }
-    const int ocol = c0w + li;
+    const int ocol = c0 + 16 * ct + li;
     if (live && ocol < a.ncols) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int row = r0 + 4 * g + j;
+            const int row = r0 + 16 * rt + 4 * g + j;
             if (row >= a.rows) continue;
             const size_t o = (size_t)ocol * a.rows + row;
             a.y[o] = a.resid ? a.resid[o] + acc[j] : acc[j];
@@ -564,21 +577,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))
     }
 }
 
-template <typename K>
-int launch_staged(K kernel, int bytes, const GemmArgs &ga, hipStream_t stream, const char *what) {
-    const dim3 grid((unsigned)((ga.rows + 15) / 16), (unsigned)((ga.ncols + 63) / 64));
-    const size_t lds = (size_t)bytes * GEMM_STAGES;
-    if (lds > 64 * 1024) { // once per kernel and process: allow the ring's dynamic LDS (up to the CU's 160 KB)
-        static std::atomic<bool> raised{false};
-        if (!raised.load()) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return fail(AQ_EHIP, what);
-            raised.store(true);
-        }
+template <int T>
+int launch_q8_gemm(const GemmArgs &ga, hipStream_t stream) {
+    static std::atomic<uint64_t> raised{0}; // per device: the ring's dynamic LDS allowed
+    int dev = 0;
+    AQ_HIP(hipGetDevice(&dev));
+    constexpr int lds = Q8Stage<T>::BYTES * Q8Stage<T>::RING;
+    if (!(raised.load() & (1ull << (dev & 63)))) {
+        AQ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(q8_gemm_kernel<T>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+        raised.fetch_or(1ull << (dev & 63));
     }
-    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, ga);
-    return hipGetLastError() == hipSuccess ? 0 : fail(AQ_EHIP, what);
+    const dim3 grid((unsigned)((ga.rows + 31) / 32), (unsigned)((ga.ncols + 63) / 64));
+    hipLaunchKernelGGL(q8_gemm_kernel<T>, grid, dim3(512), lds, stream, ga);
+    return hipGetLastError() == hipSuccess ? 0 : fail(AQ_EHIP, "q8_gemm launch");
 }
 
 template <int T, int CT>
@@ -645,10 +657,8 @@ int launch_gemm(const Weight &w, const Act &x, size_t ncols, float *y, const flo
     AQ_REQUIRE(w.cols % 256 == 0, "gemm: Q8_0 / Q4_0 columns must be a multiple of 256");
     ga.xq = x.q0;
     ga.xd = x.d0;
-    ga.xs0 = x.s0;
-    if (w.type == AQ_TYPE_Q8_0)
-        return launch_staged(q8_gemm_kernel<AQ_TYPE_Q8_0>, Q8Stage<AQ_TYPE_Q8_0>::BYTES, ga, stream, "q8_gemm launch");
-    return launch_staged(q8_gemm_kernel<AQ_TYPE_Q4_0>, Q8Stage<AQ_TYPE_Q4_0>::BYTES, ga, stream, "q8_gemm launch");
+    if (w.type == AQ_TYPE_Q8_0) return launch_q8_gemm<AQ_TYPE_Q8_0>(ga, stream);
+    return launch_q8_gemm<AQ_TYPE_Q4_0>(ga, stream);
 }
 
 } // namespace aq
