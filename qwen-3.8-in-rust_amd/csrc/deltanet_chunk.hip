@@ -142,12 +142,8 @@ __device__ __forceinline__ float from_lane7(float v) {
 
 // Work-group (head, 32 columns): wave w columns 8 w .. 8 w + 7, lane = column * 8 + key part. deltanet.rs:43-86 per row:
 // S *= decay; kv = sum_k S k; delta = (v - kv) beta; S += k delta; o = sum_k S q. The next row's inputs are loaded while
-// this one's sums run. RAW: the isolated recurrence of a verify batch, inputs as given (4-byte aligned) and the state
-// written as it stands after row a.keep - 1 (keep 0: not at all) - one launch over 192 work-groups at 48 heads x 128 x 128,
-// where the heads' own work-groups ran every row and then the kept ones again: 10.5 us for 4 rows instead of 17.
-typedef float dn_f4u __attribute__((ext_vector_type(4), aligned(4)));
-
-template <int DK, bool RAW>
+// this one's sums run.
+template <int DK>
 __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
     constexpr int KH = DK / 8;
     const DnPre p = dn_pre(a);
@@ -160,13 +156,89 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
 #pragma unroll
     for (int u = 0; u < KH; u++) s[u] = srec[(size_t)u * dv];
     auto load = [&](int b, int i) {
-        const size_t at = (size_t)kh * DK + j * KH, e = (size_t)i * a.nv + h;
-        const float *qs = RAW ? a.rq + (size_t)i * p.kd + at : p.qkv + (size_t)i * p.cd + at;
-        const float *ks = RAW ? a.rk + (size_t)i * p.kd + at : p.qkv + (size_t)i * p.cd + p.kd + at;
+        const float *row = p.qkv + (size_t)i * p.cd;
+        const float *qs = row + kh * DK + j * KH, *ks = row + p.kd + kh * DK + j * KH;
         if constexpr (KH % 4 == 0) {
 #pragma unroll
             for (int u = 0; u < KH; u += 4) {
-                const dn_f4u q4 = *reinterpret_cast<const dn_f4u *>(qs + u), k4 = *reinterpret_cast<const dn_f4u *>(ks + u);
+                const float4 q4 = *reinterpret_cast<const float4 *>(qs + u), k4 = *reinterpret_cast<const float4 *>(ks + u);
+                q[b][u] = q4.x;
+                q[b][u + 1] = q4.y;
+                q[b][u + 2] = q4.z;
+                q[b][u + 3] = q4.w;
+                k[b][u] = k4.x;
+                k[b][u + 1] = k4.y;
+                k[b][u + 2] = k4.z;
+                k[b][u + 3] = k4.w;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < KH; u++) {
+                q[b][u] = qs[u];
+                k[b][u] = ks[u];
+            }
+        }
+        v[b] = row[2 * p.kd + h * dv + c];
+        de[b] = p.decay[(size_t)i * a.nv + h];
+        be[b] = p.beta[(size_t)i * a.nv + h];
+    };
+    auto step = [&](int b, int i) {
+        float x[KH];
+#pragma unroll
+        for (int u = 0; u < KH; u++) {
+            s[u] *= de[b];
+            x[u] = s[u] * k[b][u];
+        }
+        const float kv = lane_chain<KH>(x);
+        const float delta = from_lane7((v[b] - kv) * be[b]); // lane 7 holds the sum, and its own v and beta
+#pragma unroll
+        for (int u = 0; u < KH; u++) {
+            s[u] += k[b][u] * delta;
+            x[u] = s[u] * q[b][u];
+        }
+        const float o = lane_chain<KH>(x);
+        if (j == 7) a.out[(size_t)i * p.vd + h * dv + c] = o;
+    };
+    load(0, 0);
+    int i = 0;
+    for (; i + 1 < a.t; i += 2) {
+        load(1, i + 1);
+        step(0, i);
+        load(0, i + 2 < a.t ? i + 2 : a.t - 1);
+        step(1, i + 1);
+    }
+    if (i < a.t) step(0, i);
+#pragma unroll
+    for (int u = 0; u < KH; u++) srec[(size_t)u * dv] = s[u];
+}
+
+// The isolated recurrence of a verify batch: inputs as given (4-byte aligned), the state written as it stands after row
+// a.keep - 1 (keep 0: not at all), the work split as above: one launch over 192 work-groups at 48 heads x 128 x 128, where
+// the heads' own work-groups ran every row and then the kept ones again: 10.4 us for 4 rows instead of 17. (One kernel
+// for both kept the chunk's loads from overlapping its sums: 70 us per 64 rows instead of 55.)
+typedef float dn_f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int DK>
+__global__ void __launch_bounds__(256) dn_raw_kernel(DnArgs a) {
+    constexpr int KH = DK / 8;
+    const DnPre p = dn_pre(a);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dv = a.dv;
+    const int ncb = (dv + 31) / 32, h = (int)blockIdx.x / ncb, c0 = ((int)blockIdx.x % ncb) * 32 + wave * 8;
+    if (c0 >= dv) return; // whole waves: dv is a multiple of 8
+    const int c = c0 + (lane >> 3), j = lane & 7, kh = h % a.nk;
+    float *srec = a.rec + ((size_t)h * DK + j * KH) * dv + c;
+    float s[KH], k[2][KH], q[2][KH], v[2], de[2], be[2];
+#pragma unroll
+    for (int u = 0; u < KH; u++) s[u] = srec[(size_t)u * dv];
+    auto load = [&](int b, int i) {
+        const size_t at = (size_t)kh * DK + j * KH, e = (size_t)i * a.nv + h;
+        const float *qs = a.rq + (size_t)i * p.kd + at;
+        const float *ks = a.rk + (size_t)i * p.kd + at;
+        if constexpr (KH % 4 == 0) {
+#pragma unroll
+            for (int u = 0; u < KH; u += 4) {
+                const dn_f4u q4 = *reinterpret_cast<const dn_f4u *>(qs + u);
+                const dn_f4u k4 = *reinterpret_cast<const dn_f4u *>(ks + u);
 #pragma unroll
                 for (int w = 0; w < 4; w++) {
                     q[b][u + w] = q4[w];
@@ -180,15 +252,9 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
                 k[b][u] = ks[u];
             }
         }
-        if constexpr (RAW) {
-            v[b] = a.rv[(size_t)i * p.vd + h * dv + c];
-            de[b] = exp_f(a.rg[e]);
-            be[b] = a.rbeta[e];
-        } else {
-            v[b] = p.qkv[(size_t)i * p.cd + 2 * p.kd + h * dv + c];
-            de[b] = p.decay[e];
-            be[b] = p.beta[e];
-        }
+        v[b] = a.rv[(size_t)i * p.vd + h * dv + c];
+        de[b] = exp_f(a.rg[e]);
+        be[b] = a.rbeta[e];
     };
     auto store = [&]() {
 #pragma unroll
@@ -210,7 +276,7 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
         }
         const float o = lane_chain<KH>(x);
         if (j == 7) a.out[(size_t)i * p.vd + h * dv + c] = o;
-        if (RAW && i + 1 == a.keep) store();
+        if (i + 1 == a.keep) store();
     };
     load(0, 0);
     int i = 0;
@@ -221,18 +287,17 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
         step(1, i + 1);
     }
     if (i < a.t) step(0, i);
-    if (!RAW) store();
 }
 
 template <bool RAW>
 bool launch_recurrence(const DnArgs &a, hipStream_t stream) {
     const dim3 grid((unsigned)(a.nv * ((a.dv + 31) / 32)));
     switch (a.dk) {
-    case 8: hipLaunchKernelGGL((dn_recurrence_kernel<8, RAW>), grid, dim3(256), 0, stream, a); return true;
-    case 16: hipLaunchKernelGGL((dn_recurrence_kernel<16, RAW>), grid, dim3(256), 0, stream, a); return true;
-    case 32: hipLaunchKernelGGL((dn_recurrence_kernel<32, RAW>), grid, dim3(256), 0, stream, a); return true;
-    case 64: hipLaunchKernelGGL((dn_recurrence_kernel<64, RAW>), grid, dim3(256), 0, stream, a); return true;
-    case 128: hipLaunchKernelGGL((dn_recurrence_kernel<128, RAW>), grid, dim3(256), 0, stream, a); return true;
+    case 8: hipLaunchKernelGGL((RAW ? dn_raw_kernel<8> : dn_recurrence_kernel<8>), grid, dim3(256), 0, stream, a); return true;
+    case 16: hipLaunchKernelGGL((RAW ? dn_raw_kernel<16> : dn_recurrence_kernel<16>), grid, dim3(256), 0, stream, a); return true;
+    case 32: hipLaunchKernelGGL((RAW ? dn_raw_kernel<32> : dn_recurrence_kernel<32>), grid, dim3(256), 0, stream, a); return true;
+    case 64: hipLaunchKernelGGL((RAW ? dn_raw_kernel<64> : dn_recurrence_kernel<64>), grid, dim3(256), 0, stream, a); return true;
+    case 128: hipLaunchKernelGGL((RAW ? dn_raw_kernel<128> : dn_recurrence_kernel<128>), grid, dim3(256), 0, stream, a); return true;
     }
     return false;
 }
