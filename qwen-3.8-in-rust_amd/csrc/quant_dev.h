@@ -134,8 +134,10 @@ __device__ __forceinline__ void q8k_block_wave(const float x[4], int lane, int8_
         const float iscale = -127.0f / maxv;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
+            // the code as the stored byte holds it, for the other forms and the sums too: below a max of 127 / FLT_MAX
+            // iscale is infinite and a code of -inf wraps to 0
             const int qi = (int)__builtin_rintf(iscale * x[j]);
-            q[j] = qi < 127 ? qi : 127;
+            q[j] = (int8_t)(qi < 127 ? qi : 127);
         }
         if (lane == 0) {
             const float d = 1.0f / iscale;

@@ -2,7 +2,7 @@
 column tiles with a ragged last one, rows that end inside a 4-row weight tile or a 16-row tile, fewer super-blocks than
 the LDS ring has stages, and row counts whose last pass over the CUs runs one column tile per work-group. And the
 largest integers the matrix-core sums must hold exactly: random weight bytes and every code of one sign at its largest,
-against activations of +-127 codes."""
+against activations of +-127 codes. And activation blocks too small for a finite scale."""
 import os
 import sys
 
@@ -73,3 +73,24 @@ def test_largest_sums(ctx, t, fill):
     x[1::3] *= -3.0
     x[2::3, ::2] *= -1.0
     check(ctx, t, rows, cols, raw.reshape(-1), x)
+
+
+@pytest.mark.parametrize("t", KQ)
+@pytest.mark.parametrize("n", [9, 37, 64])
+def test_tiny_activations(ctx, t, n):
+    """Blocks whose largest magnitude is so small that -127 / max overflows (below about 3.7e-37: the reference's codes
+    wrap to zero and d is zero), and on the other side of it, subnormal d: alone in a column, where the output shows
+    them, and beside ordinary blocks."""
+    rows, cols = 40, 1024
+    print(f"gemm tiny activations type {t} N={n}", flush=True)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    sizes = np.array([1e-42, 1e-39, 1e-38, 3e-37, 3.6e-37, 3.8e-37, 1e-36, 1e-34], np.float32)
+    for c in range(n):  # each column: all blocks of one size, every other block, or one block
+        for b in range(c % 3 // 2 * 2, 4 if c % 3 < 2 else 3, 1 + c % 3 % 2):
+            blk = x[c, b * 256:(b + 1) * 256]
+            x[c, b * 256:(b + 1) * 256] = blk / np.abs(blk).max() * sizes[c % len(sizes)]
+    x[:, ::7] = 0.0  # (0 times an infinite scale)
+    raw = random_blocks(t, rows, cols, 11 * n + t)
+    assert np.isfinite(O.matmul(t, raw, rows, cols, x, threads=8)).all()
+    check(ctx, t, rows, cols, raw, x)
