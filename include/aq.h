@@ -209,7 +209,8 @@ int aq_sampler_kept(aq_sampler *sp, uint32_t *ids, float *probs, size_t cap, siz
 /* `draw` (sample.rs:239-251) from the last kept set; `sample` (254-257) = process then draw. */
 int aq_sampler_draw(aq_sampler *sp, uint32_t *tok);
 int aq_sampler_sample(aq_sampler *sp, const float *logits_dev, uint32_t *tok);
-/* `write_dense` (sample.rs:259-265): the last kept set as vocab f32 at dense_dev, zeros elsewhere. */
+/* `write_dense` (sample.rs:259-265): the last kept set as vocab f32 at dense_dev, zeros elsewhere; after the work queued
+ * before the call on the context's stream and on the null stream. */
 int aq_sampler_write_dense(aq_sampler *sp, float *dense_dev);
 /* `accept_or_resample` (sample.rs:272-303): accept draft d with probability min(1, p(d)/q(d)), else a draw from
  * norm(max(0, p - q)); q_dev is the dense draft distribution (vocab f32). Greedy: accepted iff d is the argmax. */

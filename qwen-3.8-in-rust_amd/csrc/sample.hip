@@ -806,6 +806,9 @@ int aq_sampler_write_dense(aq_sampler *sp, float *dense_dev) {
     hipStream_t st = sp->ctx->stream;
     const int rc = join(sp, st);
     if (rc) return rc;
+    // the row is the caller's: what they queued on the null stream (a framework's fill of it) comes before it, as before
+    // a copy; the context's stream does not wait for that stream by itself
+    AQ_HIP(hipStreamSynchronize(nullptr));
     const int vocab = (int)sp->vocab;
     hipLaunchKernelGGL(dense_zero_kernel, dim3((vocab + 255) / 256), dim3(256), 0, st, dense_dev, vocab);
     hipLaunchKernelGGL(dense_scatter_kernel, dim3(std::min((vocab + 255) / 256, 64)), dim3(256), 0, st, dense_dev, vocab,

@@ -2,6 +2,7 @@
 edges of the 4096-key chunks, top_k at the ends of each form's range (1..128 by a bound, 129..512 by whole sorts), rows in
 ascending and descending order and rows of few distinct values (the bound leaves more keys than are sorted, so the chunk
 is sorted whole), infinities. Bar: the kept ids and probabilities and the dense row are the oracle's, bit for bit."""
+import ctypes as C
 import os
 import sys
 
@@ -47,5 +48,34 @@ def test_first_candidates_equal_the_oracle(vocab, top_k):
                               np.asarray(os_.write_dense(), np.float32).view(np.uint32)), f"row {r}: dense row"
         assert ds.draw() == os_.draw()
     for b in (lb, qb):
+        b.free()
+    ds.free()
+
+
+def test_dense_row_after_queued_writes_to_its_buffer():
+    """A row written while fills of the same buffer (and long ones before them) are still queued on the null stream, as a
+    framework that clears its tensor leaves them, and on the context's stream: the row comes after them."""
+    vocab, big = 70000, 256 << 20
+    ctx = aq.Context(0)
+    cfg = dict(temperature=0.9, top_k=40, seed=7)
+    ds, os_ = aq.Sampler(ctx, aq.sampler_config(**cfg), vocab), O.Sampler(O.sampler_config(**cfg), vocab)
+    lb, qb, long_ = aq.DeviceBuffer(ctx, vocab * 4), aq.DeviceBuffer(ctx, vocab * 4), aq.DeviceBuffer(ctx, big)
+    row = rows_of(vocab)[0]
+    lb.upload(row)
+    ds.process(lb)
+    os_.process(row)
+    want = np.asarray(os_.write_dense(), np.float32)
+    with open("/proc/self/maps") as f:  # the HIP runtime that the library runs on
+        hip = C.CDLL(next(p for p in (line.split()[-1] for line in f) if "libamdhip64" in p))
+    hip.hipMemsetAsync.argtypes = [C.c_void_p, C.c_int, C.c_size_t, C.c_void_p]
+    for i in range(3):
+        print(f"case dense row behind queued fills {i}", flush=True)
+        for _ in range(100):
+            assert hip.hipMemsetAsync(long_.p, i, big, None) == 0
+        assert hip.hipMemsetAsync(qb.p, 0x41, vocab * 4, None) == 0
+        ds.write_dense(qb)
+        assert hip.hipStreamSynchronize(C.c_void_p(None)) == 0
+        assert np.array_equal(qb.download(np.float32, vocab).view(np.uint32), want.view(np.uint32))
+    for b in (lb, qb, long_):
         b.free()
     ds.free()
