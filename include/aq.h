@@ -370,9 +370,10 @@ int aq_layer_run(aq_ctx *ctx, const aq_model_config *cfg, const aq_tensor *tenso
 int aq_deltanet_verify_commit(aq_ctx *ctx, uint32_t nk, uint32_t nv, uint32_t dk, uint32_t dv, size_t t, size_t keep,
                               const float *q, const float *k, const float *v, const float *g, const float *beta,
                               float *state_dev, float *out);
-/* The same on device arrays (q_dev .. beta_dev as above, out_dev t x nv*dv): nothing allocated or copied, the two
- * launches queued on the context's stream, which is synchronised before the call returns. t is one verify batch
- * (1..8), as for the host form. */
+/* The same on device arrays (q_dev .. beta_dev as above, out_dev t x nv*dv): one launch queued on the context's stream,
+ * which is synchronised before the call returns. out_dev may be v_dev; where it shares memory with q_dev, k_dev, g_dev,
+ * beta_dev or a part of v_dev, the output passes through a buffer allocated for the call, else nothing is allocated or
+ * copied. t is one verify batch (1..8), as for the host form. */
 int aq_deltanet_verify_commit_dev(aq_ctx *ctx, uint32_t nk, uint32_t nv, uint32_t dk, uint32_t dv, size_t t,
                                   size_t keep, const float *q_dev, const float *k_dev, const float *v_dev,
                                   const float *g_dev, const float *beta_dev, float *state_dev, float *out_dev);

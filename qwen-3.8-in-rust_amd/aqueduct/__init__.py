@@ -689,7 +689,8 @@ def deltanet_verify_commit(ctx: Context, nk, nv, dk, dv, keep, q, k, v, g, beta,
 
 
 def deltanet_verify_commit_dev(ctx: Context, nk, nv, dk, dv, t, keep, q, k, v, g, beta, state, out):
-    """aq_deltanet_verify_commit_dev: the same on DeviceBuffers (q, k, v, g, beta, state, out), nothing allocated."""
+    """aq_deltanet_verify_commit_dev: the same on DeviceBuffers (q, k, v, g, beta, state, out), nothing allocated
+    unless out lies over q, k, g, beta or a part of v."""
     check(lib().aq_deltanet_verify_commit_dev(ctx.h, nk, nv, dk, dv, t, keep, q.p, k.p, v.p, g.p, beta.p, state.p,
                                               out.p))
 

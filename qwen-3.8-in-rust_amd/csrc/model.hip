@@ -1648,8 +1648,24 @@ int aq_deltanet_verify_commit_dev(aq_ctx *ctx, uint32_t nk, uint32_t nv, uint32_
     d.t = (int)t;
     d.keep = (int)keep;
     d.out = out_dev;
+    // A head's columns are spread over work-groups that all read the head's q and k rows, so an output over the inputs'
+    // memory is formed beside it and copied. (Over v itself no: the wave that writes an element is the one that reads it,
+    // and has read it by then.)
+    const size_t n_qk = t * nk * dk, n_out = t * nv * dv, n_g = t * nv;
+    auto over = [&](const float *p, size_t n) {
+        return (uintptr_t)p < (uintptr_t)(out_dev + n_out) && (uintptr_t)out_dev < (uintptr_t)(p + n);
+    };
+    float *beside = nullptr;
+    if (over(q_dev, n_qk) || over(k_dev, n_qk) || over(g_dev, n_g) || over(beta_dev, n_g) ||
+        (v_dev != out_dev && over(v_dev, n_out))) {
+        if (dev_malloc(&beside, n_out * sizeof(float)) != hipSuccess) return fail(AQ_ENOMEM, "deltanet: output");
+        d.out = beside;
+    }
     int rc = launch_dn_raw(d, ctx->stream);
+    if (beside && !rc && hipMemcpyAsync(out_dev, beside, n_out * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+        rc = fail(AQ_EHIP, "deltanet: output copy");
     if (hipStreamSynchronize(ctx->stream) != hipSuccess && !rc) rc = fail(AQ_EHIP, "deltanet: sync");
+    if (beside) (void)hipFree(beside);
     return rc;
 }
 
