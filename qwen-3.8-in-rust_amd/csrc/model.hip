@@ -1069,8 +1069,9 @@ int aq_state_new(aq_model *m, uint32_t spec_k, uint32_t max_pos, aq_state **out)
     }
     // score rows in device memory for contexts the split core takes (head_dim of whole 64s), or that can outgrow the
     // single-launch core's LDS (the MTP's cache is the longest: cap + T rows): a prompt chunk's rows, fewer where
-    // those pass 192 MB, a verify batch's at least
-    if ((cap + 2 * T >= (size_t)ATTN_SPLIT_MIN && c.head_dim % 64 == 0) || cap + 2 * T > attn_lds_positions((int)c.head_dim)) {
+    // those pass 192 MB, a verify batch's at least. (No heads: refused below, where the buffers are made.)
+    if (c.n_head > 0 && ((cap + 2 * T >= (size_t)ATTN_SPLIT_MIN && c.head_dim % 64 == 0) ||
+                         cap + 2 * T > attn_lds_positions((int)c.head_dim))) {
         s->attn_sc_stride = (cap + 2 * T + 63) / 64 * 64;
         const size_t fit = ((size_t)192 << 20) / (c.n_head * s->attn_sc_stride * sizeof(float));
         s->attn_sc_rows = fit < T ? T : (fit > TP ? TP : fit);

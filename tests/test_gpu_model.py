@@ -156,6 +156,21 @@ def test_layer_pieces_match_oracle_and_fixtures(ctx, name, kind):
         budget_check(f"{name} step vs fixture", yg1, farr(c["step"]["y"]).reshape(yg1.shape), width)
 
 
+@pytest.mark.parametrize("name,kind", [("deltanet_layer", 0), ("mlp_layer", 2), ("attention_layer", 1)])
+@pytest.mark.parametrize("start", [0, 300, 20000])
+def test_a_config_without_heads_is_refused(ctx, name, kind, start):
+    """An error code at every position (the score rows are sized by the head count)."""
+    print(f"case {name} without heads at {start}", flush=True)
+    c = fcase(name)
+    p = Pair(ctx, c, kind)
+    p.gcfg.n_head = p.gcfg.n_head_kv = 0
+    p.gcfg.head_dim = 64
+    kv = np.zeros(64, np.float32)
+    x = farr(c["prefill"]["x"]).reshape(-1, CFG["hidden_size"])[:2]
+    with pytest.raises(aq.AqError):
+        aq.layer_run(ctx, p.gcfg, p.tensors, kind, x, start, p.g["conv"], p.g["rec"], kv, kv, 0, 16)
+
+
 def test_attention_past_the_lds_context(ctx):
     """A KV cache longer than the attention kernel's LDS holds scores for (16k positions less head_dim): the score
     rows go to device memory, with the same arithmetic, against the oracle."""
