@@ -3,8 +3,9 @@ against the CPU oracle, bit for bit: whole models of one attention layer in four
 downstream of an attention output would show a difference.
 
 Sizes are where the kernels' paths change: contexts on both sides of the split's first position and of its 64-position
-tiles, launches of 1, 4 and 8 rows and of whole prompt chunks, 2 and 6 query heads per K/V head, head_dim 64 and 256,
-a softmax row of more than one 8192-value piece."""
+tiles, launches of 1, 4 and 8 rows and of whole and ragged prompt chunks, one to eight K/V heads with 1, 2, 3, 4 and 6
+query heads each, head_dim 64, 128, 192 and 256, both forms of the weighted sum with more than one K/V head, a softmax
+row of more than one 8192-value piece, and chunks in pieces of fewer rows (few score rows: states of long contexts)."""
 import os
 import sys
 
@@ -50,10 +51,10 @@ def same(a, b):
     return np.array_equal(np.asarray(a, np.float32).view(np.uint32), np.asarray(b, np.float32).view(np.uint32))
 
 
-def check(which, n, k, rounds):
+def check(which, n, k, rounds, max_pos=None):
     cfg, gm, om = which
     ids = np.random.default_rng(n).integers(0, cfg.vocab, n).astype(np.uint32)
-    g, o = aq.State(gm, k, n + 200), O.State(om, k, n + 200)
+    g, o = aq.State(gm, k, max_pos or n + 200), O.State(om, k, n + 200)
     if k == 0:
         (ga, gl), (oa, ol) = g.prefill(ids, want_logits=True), o.prefill(ids, want_logits=True)
         assert ga == oa and same(gl, ol), "prompt logits"
@@ -86,3 +87,39 @@ def test_six_heads_of_256(wide, n, k, rounds):
 def test_softmax_rows_of_more_than_one_piece(tiny):
     print("split attention: 8,300 positions", flush=True)
     check(tiny, 8300, 3, 2)
+
+
+@pytest.fixture(scope="module")
+def heads(ctx):
+    """Models by (n_head, n_head_kv, head_dim), one at a time."""
+    made = {}
+
+    def get(nh, nkv, hd):
+        if (nh, nkv, hd) not in made:
+            made.clear()
+            made[nh, nkv, hd] = models(ctx, vocab=512, n_head=nh, n_head_kv=nkv, head_dim=hd, rope_dim=64)
+        return made[nh, nkv, hd]
+
+    return get
+
+
+@pytest.mark.parametrize("nh,nkv,hd,n,k,rounds", [
+    (12, 2, 256, 330, 3, 2),  # the wide weighted sum over two K/V heads, then 10 rows: wide scores, narrow sum
+    (12, 2, 256, 371, 0, 3),  # its ragged last chunk (51 rows: 306 vectors)
+    (8, 2, 128, 330, 3, 2), (8, 2, 128, 505, 0, 2),
+    (4, 4, 128, 300, 3, 2),  # one query head per K/V head
+    (12, 4, 192, 330, 3, 2), (12, 4, 192, 371, 7, 2),
+    (8, 8, 192, 371, 0, 3),  # and the wide weighted sum with it
+])
+def test_head_shapes(heads, nh, nkv, hd, n, k, rounds):
+    print(f"split attention {nh} heads on {nkv} of {hd}: prompt {n}, k {k}", flush=True)
+    check(heads(nh, nkv, hd), n, k, rounds)
+
+
+@pytest.mark.parametrize("which,max_pos,n,k", [("tiny", 400000, 400, 3), ("tiny", 1000000, 333, 0),
+                                               ("wide", 400000, 400, 3), ("wide", 200000, 371, 0)])
+def test_chunks_in_pieces(request, which, max_pos, n, k):
+    """A state of so many positions that the score rows are for fewer than a chunk's 64 rows (192 MB of them: 31, 12, 20
+    and 41 rows here): each chunk's attention runs in pieces, none of which divides it."""
+    print(f"split attention in pieces, {which}: {max_pos} positions, prompt {n}, k {k}", flush=True)
+    check(request.getfixturevalue(which), n, k, 2, max_pos)

@@ -604,10 +604,10 @@ def test_tiny_prompt_chunks_equal_token_by_token_and_oracle(ctx, tiny):
 
 
 def test_tiny_prompt_past_the_attention_lds_equals_token_by_token(ctx, tiny):
-    """A 16,400-token prompt on the tiny model, whose attention kernel keeps the scores of at most 16,288 positions
-    in LDS (head_dim 64): the chunks before that run attention over the whole chunk, the chunk that crosses it and
-    those after run it in 8-row pieces with the score rows in device memory. Logits and the whole state equal a
-    token-by-token feed of the same prompt, bit for bit (model.rs:443-461: prefill row i is forward_token on row i)."""
+    """A 16,400-token prompt on the tiny model: every chunk past 256 positions attends through the split core, its softmax
+    rows in up to three 8192-value pieces, past the 16,288 positions that the single-launch core's LDS holds for
+    head_dim 64. Logits and the whole state equal a token-by-token feed of the same prompt, bit for bit (model.rs:443-461:
+    prefill row i is forward_token on row i)."""
     n = 16400
     print(f"case tiny {n}-token prompt across the attention LDS limit", flush=True)
     prompt = np.random.default_rng(SEED + 11).integers(0, tiny["cfg"].vocab, n).astype(np.uint32)
