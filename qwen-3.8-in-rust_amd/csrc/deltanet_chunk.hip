@@ -146,6 +146,7 @@ __device__ __forceinline__ float from_lane7(float v) {
 template <int DK>
 __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
     constexpr int KH = DK / 8;
+    static_assert(KH % 4 == 0, "whole float4s of a row per lane");
     const DnPre p = dn_pre(a);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, dv = a.dv;
     const int ncb = (dv + 31) / 32, h = (int)blockIdx.x / ncb, c0 = ((int)blockIdx.x % ncb) * 32 + wave * 8;
@@ -158,25 +159,17 @@ __global__ void __launch_bounds__(256) dn_recurrence_kernel(DnArgs a) {
     auto load = [&](int b, int i) {
         const float *row = p.qkv + (size_t)i * p.cd;
         const float *qs = row + kh * DK + j * KH, *ks = row + p.kd + kh * DK + j * KH;
-        if constexpr (KH % 4 == 0) {
 #pragma unroll
-            for (int u = 0; u < KH; u += 4) {
-                const float4 q4 = *reinterpret_cast<const float4 *>(qs + u), k4 = *reinterpret_cast<const float4 *>(ks + u);
-                q[b][u] = q4.x;
-                q[b][u + 1] = q4.y;
-                q[b][u + 2] = q4.z;
-                q[b][u + 3] = q4.w;
-                k[b][u] = k4.x;
-                k[b][u + 1] = k4.y;
-                k[b][u + 2] = k4.z;
-                k[b][u + 3] = k4.w;
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < KH; u++) {
-                q[b][u] = qs[u];
-                k[b][u] = ks[u];
-            }
+        for (int u = 0; u < KH; u += 4) {
+            const float4 q4 = *reinterpret_cast<const float4 *>(qs + u), k4 = *reinterpret_cast<const float4 *>(ks + u);
+            q[b][u] = q4.x;
+            q[b][u + 1] = q4.y;
+            q[b][u + 2] = q4.z;
+            q[b][u + 3] = q4.w;
+            k[b][u] = k4.x;
+            k[b][u + 1] = k4.y;
+            k[b][u + 2] = k4.z;
+            k[b][u + 3] = k4.w;
         }
         v[b] = row[2 * p.kd + h * dv + c];
         de[b] = p.decay[(size_t)i * a.nv + h];
@@ -289,15 +282,23 @@ __global__ void __launch_bounds__(256) dn_raw_kernel(DnArgs a) {
     if (i < a.t) step(0, i);
 }
 
+// A model's key head sizes (a prompt chunk), and the smaller ones that the isolated recurrence takes as well.
 template <bool RAW>
 bool launch_recurrence(const DnArgs &a, hipStream_t stream) {
     const dim3 grid((unsigned)(a.nv * ((a.dv + 31) / 32)));
-    switch (a.dk) {
-    case 8: hipLaunchKernelGGL((RAW ? dn_raw_kernel<8> : dn_recurrence_kernel<8>), grid, dim3(256), 0, stream, a); return true;
-    case 16: hipLaunchKernelGGL((RAW ? dn_raw_kernel<16> : dn_recurrence_kernel<16>), grid, dim3(256), 0, stream, a); return true;
-    case 32: hipLaunchKernelGGL((RAW ? dn_raw_kernel<32> : dn_recurrence_kernel<32>), grid, dim3(256), 0, stream, a); return true;
-    case 64: hipLaunchKernelGGL((RAW ? dn_raw_kernel<64> : dn_recurrence_kernel<64>), grid, dim3(256), 0, stream, a); return true;
-    case 128: hipLaunchKernelGGL((RAW ? dn_raw_kernel<128> : dn_recurrence_kernel<128>), grid, dim3(256), 0, stream, a); return true;
+    if constexpr (RAW) {
+        switch (a.dk) {
+        case 8: hipLaunchKernelGGL(dn_raw_kernel<8>, grid, dim3(256), 0, stream, a); return true;
+        case 16: hipLaunchKernelGGL(dn_raw_kernel<16>, grid, dim3(256), 0, stream, a); return true;
+        case 32: hipLaunchKernelGGL(dn_raw_kernel<32>, grid, dim3(256), 0, stream, a); return true;
+        case 64: hipLaunchKernelGGL(dn_raw_kernel<64>, grid, dim3(256), 0, stream, a); return true;
+        case 128: hipLaunchKernelGGL(dn_raw_kernel<128>, grid, dim3(256), 0, stream, a); return true;
+        }
+    } else {
+        switch (a.dk) {
+        case 64: hipLaunchKernelGGL(dn_recurrence_kernel<64>, grid, dim3(256), 0, stream, a); return true;
+        case 128: hipLaunchKernelGGL(dn_recurrence_kernel<128>, grid, dim3(256), 0, stream, a); return true;
+        }
     }
     return false;
 }
