@@ -461,9 +461,12 @@ int launched(const char *what) {
 
 } // namespace
 
-// From ATTN_SPLIT_MIN positions: four launches cost what they cost at any length (four rows at 260 positions: scores
-// 8.8, softmax 4.2, weighted sum 6.0, quantiser 3.5 us = 22.5), the single-launch core 13.8 us at 64 positions, 18.1 at
-// 130, 23.6 at 200, 25.8 at 230.
+// From ATTN_SPLIT_MIN positions: the four launches after the prologue cost nearly the same at any length near there, the
+// single-launch core's time grows with it. 24 heads of 256 on 4 at 256 positions: 1 row 20.6 us (scores 8.5, softmax 3.9,
+// weighted sum 5.4, quantiser 2.8), 4 rows 22, 8 rows 23.4 against 32.5 in one launch (24.5 at 192 positions, 47 at 448);
+// 6 heads on 1 the same. In decode steps and verify batches (1, 2, 4 and 8 rows, five head shapes) the two cross between
+// 115 and 165 positions, so 256 is past it for all of them. A chunk of 64 rows: 50 us against 103; 45 against 45 with 6
+// heads on 1 K/V head. Of 16 rows: 43 against 42 at 256 positions, 51 against 62 at 448.
 bool attn_split_fits(const AttnArgs &a) {
     const auto al16 = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
     return a.gsc && a.base + a.t >= (size_t)ATTN_SPLIT_MIN && a.hd % 64 == 0 && a.stride % 4 == 0 && a.gsc_stride % 64 == 0 &&
@@ -478,7 +481,11 @@ int launch_attention_split(const AttnArgs &a, hipStream_t stream) {
     int rc;
     {
         // four vectors per wave and six waves (the 24 vectors of a --spec 3 verify; waves without vectors load); a
-        // prompt piece's many vectors take 16 per wave, four waves, so a K tile is read M / 64 times
+        // prompt piece's many vectors take 16 per wave, four waves, so a K tile is read M / 64 times. Up to 48 vectors
+        // (8 rows of 6 heads) the narrow form is always the faster (24 vectors: 10.3 against 16.9 us at 256 positions);
+        // at 384 vectors 18.8 against 18.2 at 256 positions, 42 against 27 at 1,000. In between the wide form is taken
+        // and loses up to 7 us on short contexts (96 vectors: 10.6 against 17.4 at 256 positions, 12.1 against 18.0 at
+        // 1,000).
         const bool wide = M > 48;
         const int nt = wide ? ScShape<16>::NT : ScShape<4>::NT, per = wide ? ScShape<16>::PER : ScShape<4>::PER;
         const int d = !wide && a.hd % 128 == 0 ? 128 : 64;
@@ -491,7 +498,10 @@ int launch_attention_split(const AttnArgs &a, hipStream_t stream) {
     }
     hipLaunchKernelGGL(attn_softmax_kernel, dim3((unsigned)a.nh, (unsigned)a.t), dim3(512), 0, stream, a);
     if ((rc = launched("attention softmax"))) return rc;
-    // one chain per lane until the waves outnumber the SIMDs, then eight per lane
+    // one chain per lane until the waves outnumber the SIMDs, then eight per lane: 49,152 chains (8 rows of 24 heads on 4)
+    // 5.8 us against 16.3 at 256 positions, 12.5 against 43.7 at 1,000; 393,216 (64 rows) 28.3 against 18.8 and 61
+    // against 47. Just past the line the one-chain form would still be the faster (98,304: 10.7 against 17 and 21
+    // against 44).
     rc = (size_t)M * a.nkv * a.hd > 64 * 1024 ? launch_wsum<false>(a, M, stream) : launch_wsum<true>(a, M, stream);
     if (rc) return rc;
     if ((rc = launched("attention weighted sum"))) return rc;

@@ -730,8 +730,8 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(AttnArgs a) {
 
 // Scores (sequential dot over head_dim, times scaling), softmax (softmax.rs:22-49: max, exp, 8-lane sum, divide),
 // weighted V sum (sequential over positions), times sigmoid(gate).
-// GSC: the score row lives in device memory (a.gsc) instead of LDS, for contexts past attn_lds_positions; the
-// arithmetic and its order are the same.
+// GSC: the score row lives in device memory (a.gsc) instead of LDS, for contexts past attn_lds_positions of head sizes
+// that the split core does not take (a layer piece on its own); the arithmetic and its order are the same.
 template <bool GSC>
 __global__ void __launch_bounds__(256) attn_core_kernel(AttnArgs a) {
     extern __shared__ float sm[]; // hd + (base + t, unless GSC) + 32

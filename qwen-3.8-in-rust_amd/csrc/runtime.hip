@@ -377,6 +377,8 @@ static int act_quantize(aq_act *a, int weight_type, size_t ncols, hipStream_t st
     AQ_HIP(hipSetDevice(a->ctx->device));
     if (is_kquant(weight_type) && !q8_fine()) {
         AQ_REQUIRE(a->a.n % 256 == 0, "aq_act_quantize: Q8_K needs n % 256 == 0 (matvec.rs:73-77)");
+        // the many-column form too, also for 8 columns or fewer: a later product may read more columns than this call
+        // quantised, and takes the others as earlier calls left them
         return launch_q8k_quantize(a->a, ncols, a->a.f32, a->a.n, stream);
     }
     if (is_kquant(weight_type) || weight_type == AQ_TYPE_Q8_0 || weight_type == AQ_TYPE_Q4_0) {
