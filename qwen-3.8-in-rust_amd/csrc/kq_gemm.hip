@@ -26,7 +26,9 @@
 // vector instructions per 16 x 16 x 256 step, of which 112 are the f32 chains; here ~150 per 16 x 64 x 256 step and
 // wave, 96 of them the chains). Two row tiles share the activation operands, which come through the LDS by direct copies
 // several steps ahead: a wave's loads return in order, so operands loaded straight into registers wait for the weights'
-// memory latency. It is bound by the waves' instruction issue, then by the copies. Measured, 64 columns: Q4_K
+// memory latency. Q4_K 17408 x 5120 at 64 columns: of 56 us the vector instructions are ~21 by count over the chip's
+// SIMDs, the matrix cores' ~8 beside them; two waves per SIMD with a barrier every step, the copies (~350 MB of
+// activation operands) and a last partial pass over the CUs leave the rest uncovered. Measured, 64 columns: Q4_K
 // 17408 x 5120 94 -> 56 us, Q6_K 5120 x 17408 211 -> 87, Q5_K 5120 x 6144 45 -> 26, Q4_K 10240 x 5120 -> 35; 37 columns:
 // Q6_K 5120 x 17408 208 -> 73 us.
 #include "aq_common.h"

@@ -1663,7 +1663,8 @@ int aq_deltanet_verify_commit_dev(aq_ctx *ctx, uint32_t nk, uint32_t nv, uint32_
         d.out = beside;
     }
     int rc = launch_dn_raw(d, ctx->stream);
-    if (beside && !rc && hipMemcpyAsync(out_dev, beside, n_out * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+    if (beside && !rc &&
+        hipMemcpyAsync(out_dev, beside, n_out * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
         rc = fail(AQ_EHIP, "deltanet: output copy");
     if (hipStreamSynchronize(ctx->stream) != hipSuccess && !rc) rc = fail(AQ_EHIP, "deltanet: sync");
     if (beside) (void)hipFree(beside);
